@@ -669,14 +669,19 @@ bool decode_eligible(const llapis_moe_layer * L, int32_t T) {
 }
 
 // prefill path (T > DEC_MAXT, either activation mode): tokens are processed in
-// chunks of Tc = PF_MAX_PAIRS / top_k; one chunk's scratch
+// chunks of Tc tokens; one chunk's scratch.  A chunk reads every routed
+// expert's weights, so a call is cut into as few chunks as PF_MAX_PAIRS
+// allows, of equal size (whole 64-token router tiles): 1900 tokens at top-8,
+// d_model 2816, every expert hot, take 1036 us as four 512-token chunks and
+// 566 us in one.  A workspace too small for that (one sized for a shorter
+// call) is served in chunks of PF_MIN_PAIRS / top_k tokens.
 struct PfWs {
     uint64_t probs, ids, w, ntiles, sorted, tiles, gtiles, xq, xd, xm, xh, ah, al, ydn, parts, total;
     int Tc, max_tiles, max_gtiles;
 };
-PfWs pf_ws(const llapis_moe_layer * L, int32_t T) {
+PfWs pf_layout(const llapis_moe_layer * L, int Tc) {
     PfWs w;
-    w.Tc = std::min<int>(T, PF_MAX_PAIRS / std::max(1, L->top_k));
+    w.Tc = Tc;
     const uint64_t P = (uint64_t)w.Tc * L->top_k;
     const uint64_t D = L->d_model, F = L->n_ff, NSB = L->d_model / 256;
     w.max_tiles = pf_max_tiles((int)P, L->n_expert);
@@ -700,9 +705,17 @@ PfWs pf_ws(const llapis_moe_layer * L, int32_t T) {
     return w;
 }
 
+PfWs pf_ws(const llapis_moe_layer * L, int32_t T, uint64_t ws_bytes = ~uint64_t(0)) {
+    const int K = std::max(1, L->top_k);
+    const int most = std::max(1, PF_MAX_PAIRS / K), least = std::min<int>(T, PF_MIN_PAIRS / K);
+    const int chunks = (T + most - 1) / most;
+    const PfWs w = pf_layout(L, chunks == 1 ? T : std::min(most, ((T + chunks - 1) / chunks + 63) / 64 * 64));
+    return w.total <= ws_bytes ? w : pf_layout(L, least);
+}
+
 bool prefill_eligible(const llapis_moe_layer * L, int32_t T) {
     return g_prefill.load() && T > DEC_MAXT && L->top_k >= 1 &&
-           L->top_k <= PF_MAX_PAIRS && L->n_expert <= 256 && L->k_slots <= 256 && L->n_ff <= PF_MAX_FF &&
+           L->top_k <= PF_MIN_PAIRS && L->n_expert <= 256 && L->k_slots <= 256 && L->n_ff <= PF_MAX_FF &&
            L->d_model % 256 == 0 &&
            L->n_ff % 32 == 0;
 }
@@ -801,7 +814,7 @@ int32_t llapis_moe_ffn(const llapis_moe_layer * L, const float * x, const float 
         }
     }
     if (prefill_eligible(L, T)) {
-        const PfWs pw = pf_ws(L, T);
+        const PfWs pw = pf_ws(L, T, ws_bytes);
         if (!workspace || ws_bytes < pw.total) return fail("llapis_moe_ffn: workspace too small");
         const int K = L->top_k;
         const int src = L->gelu_mode == LLAPIS_GELU_TANH ? dev::SRC_GEGLU_TANH : dev::SRC_GEGLU_TABLE;

@@ -144,21 +144,34 @@ __constant__ Iq2sSplit c_iq2s_split = make_iq2s_split();
 
 // ----------------------------------------------------------------- bucket
 
-// One workgroup.  P = T * top_k <= PF_MAX_PAIRS, n_expert <= 256.  A
-// counting sort by expert with LDS atomics: counts, an exclusive scan over
-// the experts (pair offsets and group offsets), then each pair takes the
-// next slot of its expert.  The order of pairs inside an expert's range is
-// not fixed, and need not be: each pair's output column is computed on its
-// own.
+// One workgroup of PREP_WG threads.  P = T * top_k <= PF_MAX_PAIRS, n_expert
+// <= 256.  A counting sort by expert with LDS atomics: counts, an exclusive
+// scan over the experts (pair offsets and group offsets; one wave scan and the
+// sums of the waves before it, two barriers), then each pair takes the next
+// slot of its expert.  The order of pairs inside an expert's range is not
+// fixed, and need not be: each pair's output column is computed on its own.
+// 16 waves: the ids of a long call (16384 pairs) are 16 loads a thread.
+constexpr int PREP_WG = 1024;
+
+__device__ __forceinline__ int wave_scan_incl(int v) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(v, o, 64);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+
 __device__ __forceinline__ void pf_bucket(const PfParams & p) {
-    constexpr int PER = PF_MAX_PAIRS / WG;
-    __shared__ int s_cnt[257], s_fill[257], s_off[257], s_nt[257], s_gf[256], s_gr[256], s_hot;
+    constexpr int PER = PF_MAX_PAIRS / PREP_WG;
+    __shared__ int s_cnt[257], s_fill[257], s_off[257], s_tot[4][4], s_hot;
     const int P = p.T * p.top_k, E = p.n_expert;
     __shared__ int s_se[256], s_ss[256];
     int ev[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        const int q = threadIdx.x + WG * k;
+        const int q = threadIdx.x + PREP_WG * k;
         const int v = q < P ? p.ids[q] : -1;
         ev[k] = (v >= 0 && v < E) ? v : 256;     // 256: invalid id
     }
@@ -170,15 +183,15 @@ __device__ __forceinline__ void pf_bucket(const PfParams & p) {
         s_se[e0] = p.slot_exp[e0];
         s_ss[e0] = p.slot_state[e0];
     }
-    for (int i = threadIdx.x; i < 257; i += WG) {
-        s_cnt[i] = 0;
-        s_fill[i] = 0;
+    if (threadIdx.x < 257) {
+        s_cnt[threadIdx.x] = 0;
+        s_fill[threadIdx.x] = 0;
     }
     if (threadIdx.x == 0) s_hot = 0;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < PER; ++k)
-        if (threadIdx.x + WG * k < P) atomicAdd(&s_cnt[ev[k]], 1);
+        if (threadIdx.x + PREP_WG * k < P) atomicAdd(&s_cnt[ev[k]], 1);
     __syncthreads();
     int n_e = 0, tier = 1, idx = e0;
     if (e0 < E) {
@@ -199,66 +212,70 @@ __device__ __forceinline__ void pf_bucket(const PfParams & p) {
         const int hot = tier == 0 ? n_e : 0;
         if (hot) atomicAdd(&s_hot, hot);
     }
-    s_off[threadIdx.x] = n_e;
-    s_nt[threadIdx.x] = nt_e;
-    s_gf[threadIdx.x] = gf_e;
-    s_gr[threadIdx.x] = gr_e;
-    __syncthreads();
-    for (int o = 1; o < 256; o <<= 1) {          // inclusive scans over the experts
-        const int a = threadIdx.x >= o ? s_off[threadIdx.x - o] : 0;
-        const int b = threadIdx.x >= o ? s_nt[threadIdx.x - o] : 0;
-        const int c = threadIdx.x >= o ? s_gf[threadIdx.x - o] : 0;
-        const int d = threadIdx.x >= o ? s_gr[threadIdx.x - o] : 0;
-        __syncthreads();
-        s_off[threadIdx.x] += a;
-        s_nt[threadIdx.x] += b;
-        s_gf[threadIdx.x] += c;
-        s_gr[threadIdx.x] += d;
-        __syncthreads();
-    }
-    const int pair0 = s_off[threadIdx.x] - n_e, tile0 = s_nt[threadIdx.x] - nt_e;
-    const int total = s_off[255], tiles = min(s_nt[255], p.max_tiles);
-    const int nfull = s_gf[255], gf0 = s_gf[threadIdx.x] - gf_e, gr0 = nfull + s_gr[threadIdx.x] - gr_e;
-    for (int b = 0; b <= gf_e; ++b) {
-        const int gi = b < gf_e ? gf0 + b : gr0;
-        if ((b == gf_e && !gr_e) || gi >= p.max_gtiles) continue;
-        PfTile t;
-        t.tier = tier;
-        t.idx = idx;
-        t.begin = pair0 + b * gcap;
-        t.n = min(gcap, n_e - b * gcap);
-        p.gtiles[gi] = t;
-    }
-    if (p.rc_hits && threadIdx.x == 0) {
-        atomicAdd(p.rc_hits, s_hot);
-        atomicAdd(p.rc_hits + 1, P - s_hot);
+    // inclusive scans over the experts (waves 0..3)
+    const int wave = threadIdx.x >> 6;
+    int c_off = wave_scan_incl(n_e), c_nt = wave_scan_incl(nt_e), c_gf = wave_scan_incl(gf_e), c_gr = wave_scan_incl(gr_e);
+    if (wave < 4 && (threadIdx.x & 63) == 63) {
+        s_tot[wave][0] = c_off;
+        s_tot[wave][1] = c_nt;
+        s_tot[wave][2] = c_gf;
+        s_tot[wave][3] = c_gr;
     }
     __syncthreads();
-    s_off[threadIdx.x] = pair0;
+    int total[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        if (w < wave) {
+            c_off += s_tot[w][0];
+            c_nt += s_tot[w][1];
+            c_gf += s_tot[w][2];
+            c_gr += s_tot[w][3];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) total[i] += s_tot[w][i];
+    }
+    const int pair0 = c_off - n_e, tile0 = c_nt - nt_e, nfull = total[2], gf0 = c_gf - gf_e, gr0 = nfull + c_gr - gr_e;
+    if (e0 < E) {
+        s_off[e0] = pair0;
+        for (int b = 0; b <= gf_e; ++b) {
+            const int gi = b < gf_e ? gf0 + b : gr0;
+            if ((b == gf_e && !gr_e) || gi >= p.max_gtiles) continue;
+            PfTile t;
+            t.tier = tier;
+            t.idx = idx;
+            t.begin = pair0 + b * gcap;
+            t.n = min(gcap, n_e - b * gcap);
+            p.gtiles[gi] = t;
+        }
+        for (int b = 0; b < nt_e; ++b) {
+            if (tile0 + b >= p.max_tiles) break;
+            PfTile t;
+            t.tier = tier;
+            t.idx = idx;
+            t.begin = pair0 + b * PF_TOK;
+            t.n = min(PF_TOK, n_e - b * PF_TOK);
+            p.tiles[tile0 + b] = t;
+        }
+    }
     if (threadIdx.x == 0) {
-        s_off[256] = total;                     // invalid ids are placed after every expert's pairs
-        *p.n_tiles = tiles;
-        *p.n_gtiles = min(nfull + s_gr[255], p.max_gtiles);
-    }
-    for (int b = 0; b < nt_e; ++b) {
-        if (tile0 + b >= p.max_tiles) break;
-        PfTile t;
-        t.tier = tier;
-        t.idx = idx;
-        t.begin = pair0 + b * PF_TOK;
-        t.n = min(PF_TOK, n_e - b * PF_TOK);
-        p.tiles[tile0 + b] = t;
+        s_off[256] = total[0];                  // invalid ids are placed after every expert's pairs
+        *p.n_tiles = min(total[1], p.max_tiles);
+        *p.n_gtiles = min(nfull + total[3], p.max_gtiles);
+        if (p.rc_hits) {
+            atomicAdd(p.rc_hits, s_hot);
+            atomicAdd(p.rc_hits + 1, P - s_hot);
+        }
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        const int q = threadIdx.x + WG * k;
+        const int q = threadIdx.x + PREP_WG * k;
         if (q < P) p.sorted[s_off[ev[k]] + atomicAdd(&s_fill[ev[k]], 1)] = q;
     }
     // a pair with an invalid id is in no group: it contributes zeros to the combine
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        const int q = threadIdx.x + WG * k;
+        const int q = threadIdx.x + PREP_WG * k;
         if (q < P && ev[k] == 256)
             for (int r = 0; r < p.d_model; ++r) p.ydn[(int64_t)q * p.d_model + r] = 0.0f;
     }
@@ -270,10 +287,10 @@ __device__ __forceinline__ void pf_bucket(const PfParams & p) {
 // values, the scale, and the 8 per-32 sums as {hi_0..hi_7, lo_0..lo_7} with
 // sum = 32 hi + lo, 0 <= lo < 32 (each part exact in fp16).
 __device__ __forceinline__ void pf_quant_x(const PfParams & p, int blk) {
-    __shared__ __align__(16) uint8_t scratch[WG / 64][512];
+    __shared__ __align__(16) uint8_t scratch[PREP_WG / 64][512];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int NSB = p.d_model / 256;
-    const int job = blk * (WG / 64) + wave;
+    const int job = blk * (PREP_WG / 64) + wave;
     const bool live = job < p.T * NSB;
     const int t = live ? job / NSB : 0, s = live ? job % NSB : 0;
     ActView L;
@@ -311,7 +328,7 @@ __device__ __forceinline__ void pf_quant_x(const PfParams & p, int blk) {
 __device__ __forceinline__ void pf_quant_x1(const PfParams & p, int blk) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int D = p.d_model, per = D / 64;
-    const int job = blk * (WG / 64) + wave;
+    const int job = blk * (PREP_WG / 64) + wave;
     if (job >= p.T * per) return;                        // whole waves leave
     const int t = job / per, pos = 64 * (job - t * per) + lane;
     const float v = p.x[(int64_t)t * D + pos];
@@ -343,7 +360,7 @@ __device__ __forceinline__ void pf_quant_x1(const PfParams & p, int blk) {
 // depends on the other), so the quantisation runs while the one bucketing
 // workgroup does and the chunk has one kernel boundary fewer.
 template <int AM>
-__global__ __launch_bounds__(WG) void k_pf_prep(const PfParams p) {
+__global__ __launch_bounds__(PREP_WG) void k_pf_prep(const PfParams p) {
     if (blockIdx.x == 0) pf_bucket(p);
     else if (AM == AM_Q8_1) pf_quant_x1(p, blockIdx.x - 1);
     else pf_quant_x(p, blockIdx.x - 1);
@@ -1555,9 +1572,10 @@ hipError_t launch_prefill(const PfParams & p0, int hgu, int cgu, int hdn, int cd
     if (ev)
         for (int i = 0; i < 4; ++i) e[i] = ev[i];
     const int NSB = p.d_model / 256;
+    constexpr int PW = PREP_WG / 64;                // token blocks per quantising workgroup
     if (p.act_mode == AM_Q8_1)
-        hipLaunchKernelGGL(k_pf_prep<AM_Q8_1>, dim3(1 + (p.T * (p.d_model / 64) + 3) / 4), dim3(WG), 0, s, p);
-    else hipLaunchKernelGGL(k_pf_prep<AM_CPU>, dim3(1 + (p.T * NSB + 3) / 4), dim3(WG), 0, s, p);
+        hipLaunchKernelGGL(k_pf_prep<AM_Q8_1>, dim3(1 + (p.T * (p.d_model / 64) + PW - 1) / PW), dim3(PREP_WG), 0, s, p);
+    else hipLaunchKernelGGL(k_pf_prep<AM_CPU>, dim3(1 + (p.T * NSB + PW - 1) / PW), dim3(PREP_WG), 0, s, p);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     {

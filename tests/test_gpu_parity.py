@@ -587,3 +587,27 @@ def test_prefill_chunks_and_generic_agree(gpu, oracle):
     check_flip_tolerant(out_p.cpu().numpy(), out_g.cpu().numpy())
     out_o, _ = oracle.moe_experts(lay, x, ids_p.cpu().numpy(), w_p.cpu().numpy())
     check_flip_tolerant(out_p.cpu().numpy(), out_o)
+
+
+def test_prefill_in_a_workspace_of_a_shorter_call(gpu):
+    """A long call is one chunk in a workspace of its own size and falls back
+    to chunks of 4096 / top_k tokens in a workspace sized for fewer tokens:
+    the same results either way, bit for bit (a pair's result depends neither
+    on its group nor on its chunk)."""
+    import ctypes as C
+    torch = torch_mod()
+    spec, T = SMALL, 1500                        # top_k 4: chunks of 1024 tokens
+    say(f"prefill T={T} in a smaller workspace")
+    dl = la.DeviceLayer(_layer_case(spec, 91, 6, True), gpu)
+    x = torch.from_numpy(tokens(601, T, spec.d_model)).to(gpu)
+    lib, d = la.lib(), dl.desc()
+    want = [t.clone() for t in dl.forward(x)]
+    ws = torch.empty(int(lib.llapis_moe_ffn_workspace_size(C.byref(d), 1024)), dtype=torch.uint8, device=gpu)
+    assert ws.numel() < int(lib.llapis_moe_ffn_workspace_size(C.byref(d), T))
+    out, ids, w = torch.empty_like(want[0]), torch.empty_like(want[1]), torch.empty_like(want[2])
+    rc = lib.llapis_moe_ffn(C.byref(d), x.data_ptr(), None, T, out.data_ptr(), ids.data_ptr(), w.data_ptr(),
+                            ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.llapis_last_error()
+    torch.cuda.synchronize()
+    for a, b in zip((out, ids, w), want):
+        assert torch.equal(a, b)
