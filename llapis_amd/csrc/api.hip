@@ -713,6 +713,12 @@ PfWs pf_ws(const llapis_moe_layer * L, int32_t T, uint64_t ws_bytes = ~uint64_t(
     return w.total <= ws_bytes ? w : pf_layout(L, least);
 }
 
+// the smallest workspace that llapis_moe_ffn accepts for T tokens on any path
+uint64_t least_workspace(const llapis_moe_layer * L, int32_t T) {
+    const uint64_t b = ffn_ws(L, T).total;
+    return std::max(b, T <= DEC_MAXT ? dec_ws(L, T).total : pf_ws(L, T, 0).total);
+}
+
 bool prefill_eligible(const llapis_moe_layer * L, int32_t T) {
     return g_prefill.load() && T > DEC_MAXT && L->top_k >= 1 &&
            L->top_k <= PF_MIN_PAIRS && L->n_expert <= 256 && L->k_slots <= 256 && L->n_ff <= PF_MAX_FF &&
@@ -731,8 +737,7 @@ void llapis_set_tuning(int32_t key, int32_t value) {
 
 uint64_t llapis_moe_ffn_workspace_size(const llapis_moe_layer * L, int32_t n_tokens) {
     if (!L || n_tokens <= 0) return 0;
-    uint64_t b = ffn_ws(L, n_tokens).total;
-    if (n_tokens <= DEC_MAXT) b = std::max(b, dec_ws(L, n_tokens).total);
+    uint64_t b = least_workspace(L, n_tokens);
     if (n_tokens > DEC_MAXT) b = std::max(b, pf_ws(L, n_tokens).total);
     return b;
 }
@@ -979,7 +984,8 @@ int32_t llapis_moe_ffn_noalloc(const llapis_moe_layer * L, const float * x, cons
                                float * out, int32_t * ids_out, float * w_out, void * stream) {
     if (!L) return fail("llapis_moe_ffn_noalloc: null layer");
     if (T <= 0) return 0;
-    const uint64_t need = llapis_moe_ffn_workspace_size(L, T);
+    // the least workspace the call runs in (a long call also takes shorter chunks)
+    const uint64_t need = least_workspace(L, T);
     if (need > LLAPIS_NOALLOC_SCRATCH_BYTES)
         return fail("llapis_moe_ffn_noalloc: this call needs " + std::to_string(need) +
                     " bytes of scratch, more than the fixed " + std::to_string(LLAPIS_NOALLOC_SCRATCH_BYTES) +

@@ -80,6 +80,20 @@ def test_noalloc_refuses_a_call_beyond_its_array(gpu):
     assert all(torch.equal(a, b) for a, b in zip(ref, got))
 
 
+def test_noalloc_takes_a_long_call_in_short_chunks(gpu):
+    """670 tokens of a small layer: the workspace of the whole call in one
+    chunk is larger than the array, that of 512-token chunks is not, so the
+    call runs in those."""
+    import torch
+    say("noalloc T=670")
+    spec = la.LayerSpec(d_model=256, n_ff=64, n_expert=16, top_k=8)
+    dl = la.DeviceLayer(_layer(spec, 65, 7), gpu)
+    assert int(la.lib().llapis_moe_ffn_workspace_size(C.byref(dl.desc()), 670)) > la._lib.NOALLOC_SCRATCH_BYTES
+    ref, got = _both(gpu, dl, tokens(67, 670, spec.d_model))
+    for a, b, what in zip(ref, got, ("out", "ids", "weights")):
+        assert torch.equal(a, b), what
+
+
 @pytest.mark.parametrize("T", [1, 4, 40])
 def test_noalloc_captured_in_a_graph(gpu, T):
     """Three llapis_moe_ffn_noalloc calls captured in one HIP graph (one
