@@ -127,7 +127,7 @@ hipError_t launch_fire(const FireParams & f, int ht, int ct, int act_mode, hipSt
 // ------------------------------------------------------------ prefill path
 
 constexpr int PF_ROWS = 128;          // weight rows per workgroup (4 waves x 32)
-constexpr int PF_TOK = 96;            // routed pairs per down group (six 16-token MFMA tiles)
+constexpr int PF_TOK = 64;            // routed pairs per down group (four 16-token MFMA tiles)
 constexpr int PF_GTOK = 128;          // routed pairs per gate_up group, at most
 constexpr int PF_MAX_PAIRS = 16384;   // routed pairs per prefill launch (T * top_k), at most
 constexpr int PF_MIN_PAIRS = 4096;    // ... that a workspace of any accepted size holds

@@ -107,6 +107,14 @@ __device__ __forceinline__ uint32_t h2bits(h2 v) {
 __device__ __forceinline__ uint32_t magic_lo(uint32_t x) { return __builtin_amdgcn_perm(0x64646464u, x, 0x04010400u); }
 __device__ __forceinline__ uint32_t magic_hi(uint32_t x) { return __builtin_amdgcn_perm(0x64646464u, x, 0x04030402u); }
 
+// group g's record (g may lie past the groups), its load issued beside the
+// count's rather than after the branch on it
+__device__ __forceinline__ PfTile load_tile(const PfTile * tiles, int max_tiles, int g) {
+    PfTile t = tiles[min(g, max_tiles - 1)];
+    asm volatile("" : "+s"(t.tier), "+s"(t.idx), "+s"(t.begin), "+s"(t.n));
+    return t;
+}
+
 __device__ __forceinline__ bool tile_valid(const PfParams & p, const PfTile & t) {
     return (t.tier == 0 && t.idx >= 0 && t.idx < p.k_slots) || (t.tier == 1 && t.idx >= 0 && t.idx < p.n_expert);
 }
@@ -371,6 +379,14 @@ __global__ __launch_bounds__(PREP_WG) void k_pf_prep(const PfParams p) {
 // the epilogue's staging of one 16-token tile: [128 rows][17]
 constexpr int GU_STP = 17;
 constexpr int GU_WREG = 5;     // weight chunks per thread per super-block (q8_1 kernel; 128 rows x 9)
+
+// Where value i of a 32-block sits in the down activations (ah, al): in the
+// order the weights come out of their dwords.  Lane quarter q of a fragment
+// takes the nibbles of qs bytes 4 q .. 4 q + 3 (low: values 4 q + j, high:
+// 16 + 4 q + j), as 16-bit pairs of bytes 0, 2 and 1, 3.
+__device__ __forceinline__ int dn_pos(int i) {
+    return 8 * ((i >> 2) & 3) + 4 * (i & 1) + 2 * (i >> 4) + ((i >> 1) & 1);
+}
 
 // q8_0 (x86 CPU build, arch/x86/quants.c:302-360) or q8_1 (ggml-cuda
 // quantize.cu:5-50) of one 32-block held one value per lane of a half-wave,
@@ -822,14 +838,13 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
         const bool live = j < tile.n && fi < F;
         const int64_t qp = L.pair[j];
         const float v = GSRC == SRC_GEGLU_TABLE ? geglu_from_entry(gv[k], uv[k], te[k]) : geglu1<GSRC>(gv[k], uv[k]);
-        q8_store32<AM_CPU>(v, p.ah + qp * F + fi + i, p.al + qp * F + fi + i, nullptr, live);
+        q8_store32<AM_CPU>(v, p.ah + qp * F + fi + dn_pos(i), p.al + qp * F + fi + dn_pos(i), nullptr, live);
     }
 }
 
-// Grid: 8 x ceil(max_tiles / 8) x RB workgroups in one dimension.  The
-// hardware deals workgroups to the 8 XCDs in turn (workgroup i to XCD
-// i mod 8), so workgroup i serves group 8 (k / RB) + i mod 8, row block
-// k mod RB (k = i / 8): all row blocks of a group run on one XCD and read
+// Grid: (8, RB, ceil(max_tiles / 8)) workgroups.  The hardware deals
+// workgroups to the 8 XCDs in turn, x first, so workgroup (x, y, z) serves
+// group 8 z + x, row block y: all row blocks of a group run on XCD x and read
 // its activations through one L2, and every XCD takes the full groups first.
 template <int HT, int CT, int GSRC>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_pf_gate_up(const PfParams p) {
@@ -844,11 +859,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     __shared__ int tok[G2_TOKMAX], pair[G2_TOKMAX];
     const Gu2Lds sm = {x0, x1, w0, w1, mb0, mb1, d80, d81, reinterpret_cast<uint2 *>(w0),
                        reinterpret_cast<u32x4 *>(w1), tok, pair};
-    const int RB = (p.n_ff + 63) / 64;
-    const int i = blockIdx.x, k = i >> 3;
-    const int g = 8 * (k / RB) + (i & 7), rb = k - (k / RB) * RB;
+    const int g = 8 * blockIdx.z + blockIdx.x, rb = blockIdx.y;
+    const PfTile tile = load_tile(p.gtiles, p.max_gtiles, g);
     if (g >= *p.n_gtiles) return;
-    const PfTile tile = p.gtiles[g];
     if (!tile_valid(p, tile) || tile.n <= 0) return;
     const int wt = tile.tier == 0 ? HT : CT;
     const int nt = (tile.n + 15) >> 4;
@@ -1227,7 +1240,7 @@ __device__ __forceinline__ void pf_gate_up_group_q1(const PfParams & p, const Pf
             const float uv = stg[(64 + 32 * blk + i) * GU_STP + tk];
             const float v = geglu1<GSRC>(gv, uv);
             const int64_t qp = sm.pair[min(j, NTOK - 1)];
-            q8_store32<AM_Q8_1>(v, p.ah + qp * F + fi + i, p.al + qp * F + fi + i, nullptr, live);
+            q8_store32<AM_Q8_1>(v, p.ah + qp * F + fi + dn_pos(i), p.al + qp * F + fi + dn_pos(i), nullptr, live);
         }
     }
 }
@@ -1238,11 +1251,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     // the gate_up groups of this mode hold <= PF_TOK1Q4 pairs of a Q4_K
     // expert, <= PF_TOK1IQ2 of an IQ2_S one; workgroups are dealt to the XCDs
     // as k_pf_gate_up's (all row blocks of a group on one)
-    const int RB = (p.n_ff + 63) / 64;
-    const int i = blockIdx.x, k = i >> 3;
-    const int g = 8 * (k / RB) + (i & 7), rb = k - (k / RB) * RB;
+    const int g = 8 * blockIdx.z + blockIdx.x, rb = blockIdx.y;
+    const PfTile tile = load_tile(p.gtiles, p.max_gtiles, g);
     if (g >= *p.n_gtiles) return;
-    const PfTile tile = p.gtiles[g];
     const bool q4 = (tile.tier == 0 ? HT : CT) == T_Q4_K;
     if (!tile_valid(p, tile) || tile.n <= 0 || tile.n > (q4 ? PF_TOK1Q4 : PF_TOK1IQ2)) return;
     const int n = tile.n;
@@ -1262,80 +1273,99 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // w owns rows 32 w .. 32 w + 31 as two 16-row MFMA tiles.  K (n_ff) runs in
 // chunks of two 32-blocks, CPS chunks a step (groups of up to 32 pairs take
 // two: a small group's step is short, and each step waits for its loads).
-// The load unit copies the next step's activation parts into LDS while the
-// current one's are used (two buffers, separately declared, one barrier per
-// step): a pair's chunk is 16 slots of 16 bytes (slots 0..7 the high parts
-// of its 64 values, 8..15 the low parts), slot s at s ^ (pair & 15), so the
-// 16 pairs of an MFMA fragment read 16 distinct slots.  Each lane loads its
-// rows' window of the step (44 bytes of Q5_0, 36 of IQ4_NL a chunk) straight
-// into registers, the next step's in flight during the current one's MFMAs.
+// The load unit copies the next step's operands into LDS while the current
+// one's are used.  Activation parts: two buffers, separately declared, one
+// barrier per step; a pair's chunk is 16 slots of 16 bytes (slots 0..7 the
+// high parts of its 64 values, 8..15 the low parts), slot s at
+// s ^ (pair & 15), so the 16 pairs of an MFMA fragment read 16 distinct
+// slots.  Weights: a wave copies its own 32 rows' window of the step, as
+// 16-byte granules (G per row, an odd count: the rows of a fragment read
+// start in different banks), and takes the fields of a step out of them into
+// registers before it starts the next step's copy into the same room.
+//
+// Why through LDS: the four quarters of a fragment share a row, so rows read
+// straight into registers are read four times, and a 16-byte load of 64
+// lanes costs the L1 64 accesses whatever lanes share: 61 million accesses a
+// 512-token chunk (dual, K = 57), 240 thousand of a CU's 290 thousand cycles.
+// With the windows in LDS 16 million, and with the fragment order of dn_pos
+// and dn_frag's fewer VALU instructions (27 against 35 million) the kernel
+// takes 92 against 122 us there (fastest dispatches, traced), 211 against 254
+// us at 1900 tokens, 26 against 34 us at 12.  It is bound by VALU issue (57 %
+// of its cycles) and the matrix cores (21 %).  Groups of 64 pairs: at 96 the
+// activation buffers leave room for two workgroups a CU instead of three.
 constexpr int D2_XB = PF_TOK * 256;                // activations of one step: [chunk][pair slot][16][16 bytes]
+constexpr int D2_WB = 4 * 1024;                    // one wave's weight windows of a step, at most (whole copies)
 
 struct Dn2Lds {
     uint8_t * x0; uint8_t * x1;
+    uint8_t * w;                                   // this wave's windows
     int * pair;
+    uint32_t * yoff;                               // byte offsets of the pairs' rows in ydn
 };
 
-// One lane's row window of a two-block chunk: 44 bytes (Q5_0) or 36
-// (IQ4_NL), from the chunk's first byte.
-struct DnWin {
-    u32x4 a, b;
-    u32x3 e;
+// One lane's fields of one block of a row: d, Q5_0's qh, and the lane's dword
+// of the nibbles.  Fields are 2-aligned; the dword ones are read as the
+// aligned dwords around them (a misaligned LDS read takes several times as
+// long) and shifted into place.
+struct DnRaw {
+    uint32_t d, qh0, qh1, qs0, qs1;
 };
-template <int I>
-__device__ __forceinline__ uint32_t win_dword(const DnWin & w) {
-    if constexpr (I < 4) return w.a[I];
-    else if constexpr (I < 8) return w.b[I - 4];
-    else return w.e[I - 8];
-}
-// the dword holding bytes BYTE .. BYTE + 3 of the window (BYTE even)
-template <int BYTE>
-__device__ __forceinline__ uint32_t win_at(const DnWin & w) {
-    if constexpr (BYTE & 3) return __builtin_amdgcn_alignbit(win_dword<(BYTE >> 2) + 1>(w), win_dword<(BYTE >> 2)>(w), 16);
-    else return win_dword<(BYTE >> 2)>(w);
-}
-
-// 8 values (8 u .. 8 u + 7 of block B of the chunk) as exact fp16 integers:
-// Q5_0 q - 16 (ggml-quants.c:442), IQ4_NL kvalues[q] (:2653); the block
-// scale d_w out.  Block 1 starts 2 bytes into a dword of the window.
-template <int T, int B>
-__device__ __forceinline__ h8 down_frag_r(const DnWin & w, int u, float & d) {
-    constexpr int BS = T == T_Q5_0 ? 22 : 18;
-    constexpr int o0 = BS * B;                          // the block's first byte
-    d = h2f((o0 & 3) ? (win_dword<(o0 >> 2)>(w) >> 16) : (win_dword<(o0 >> 2)>(w) & 0xFFFFu));
-    const bool hiq = (u & 1) != 0;                      // bytes 8..15 of the qs
-    uint32_t h[4];
+// x = the dword at byte `at` of the window's room, `at` 4-aligned
+__device__ __forceinline__ uint32_t lds_dword(const uint8_t * w, int at) { return *reinterpret_cast<const uint32_t *>(w + at); }
+template <int T>
+__device__ __forceinline__ void dn_raw_read(DnRaw & r, const uint8_t * w, int blk, int q) {
+    r.d = *reinterpret_cast<const uint16_t *>(w + blk);
+    const int a = (blk + 2) & ~3;                       // qh (Q5_0) or the first nibbles
+    constexpr int QS = T == T_Q5_0 ? 4 : 0;
     if constexpr (T == T_Q5_0) {
-        // values 0..15: low nibbles of qs[0..15]; 16..31: high nibbles
-        const uint32_t qs0 = hiq ? win_at<o0 + 14>(w) : win_at<o0 + 6>(w);
-        const uint32_t qs1 = hiq ? win_at<o0 + 18>(w) : win_at<o0 + 10>(w);
-        const uint32_t qh = __builtin_amdgcn_ubfe(win_at<o0 + 2>(w), 8 * u, 8);
-        const int sh = 4 * (u >> 1);
-        uint32_t x[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const uint32_t nib = ((i ? qs1 : qs0) >> sh) & 0x0F0F0F0Fu;
-            const uint32_t hb = (qh >> (4 * i)) & 15u;
-            x[i] = nib | (((hb * 0x00204081u) & 0x01010101u) << 4);   // bit k -> bit 4 of byte k
-        }
-        const h2 off = h2{(_Float16)(-1040.0f), (_Float16)(-1040.0f)};
-        h[0] = h2bits(as_h2(magic_lo(x[0])) + off);
-        h[1] = h2bits(as_h2(magic_hi(x[0])) + off);
-        h[2] = h2bits(as_h2(magic_lo(x[1])) + off);
-        h[3] = h2bits(as_h2(magic_hi(x[1])) + off);
-    } else {
-        const uint32_t qs0 = hiq ? win_at<o0 + 10>(w) : win_at<o0 + 2>(w);
-        const uint32_t qs1 = hiq ? win_at<o0 + 14>(w) : win_at<o0 + 6>(w);
-        const int sh = 4 * (u >> 1);
-        const h2 off = h2{(_Float16)(-1152.0f), (_Float16)(-1152.0f)};
-        uint32_t x[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) x[i] = iq4nl_lookup(((i ? qs1 : qs0) >> sh) & 0x0F0F0F0Fu) ^ 0x80808080u;
-        h[0] = h2bits(as_h2(magic_lo(x[0])) + off);
-        h[1] = h2bits(as_h2(magic_hi(x[0])) + off);
-        h[2] = h2bits(as_h2(magic_lo(x[1])) + off);
-        h[3] = h2bits(as_h2(magic_hi(x[1])) + off);
+        r.qh0 = lds_dword(w, a);
+        r.qh1 = lds_dword(w, a + 4);
     }
+    r.qs0 = lds_dword(w, a + QS + 4 * q);
+    r.qs1 = lds_dword(w, a + QS + 4 * q + 4);
+}
+
+// the fields are in their registers when this returns
+template <int T>
+__device__ __forceinline__ void dn_raw_here(DnRaw & r) {
+    if constexpr (T == T_Q5_0) asm volatile("" : "+v"(r.d), "+v"(r.qh0), "+v"(r.qh1), "+v"(r.qs0), "+v"(r.qs1));
+    else asm volatile("" : "+v"(r.d), "+v"(r.qs0), "+v"(r.qs1));
+}
+
+// The lane's 8 weights of a block times 2^-9, exact in fp16: Q5_0 q - 16
+// (ggml-quants.c:442), IQ4_NL kvalues[q] (:2653).  Each is formed as an
+// unsigned byte u (q; kvalues + 128) in the low bits of an fp16, where it
+// reads u 2^-24; one fma scales it by 2^15 and takes the offset off.
+template <int T>
+__device__ __forceinline__ h8 dn_frag(const DnRaw & r, uint32_t sh, uint32_t qrot) {
+    const uint32_t qs = __builtin_amdgcn_alignbit(r.qs1, r.qs0, sh);
+    uint32_t lo, hi;                                    // the low nibbles' four values, the high ones'
+    _Float16 off;
+    if constexpr (T == T_Q5_0) {
+        // bits 4..7: qh bits 4 q .. 4 q + 3 (the low nibbles' fifth bits), 20..23: 16 + 4 q .. (qrot = 4 q - 4)
+        const uint32_t qh = __builtin_amdgcn_alignbit(r.qh1, r.qh0, sh);
+        const uint32_t g = __builtin_amdgcn_alignbit(qh, qh, qrot);
+        lo = (qs & 0x0F0F0F0Fu) | (__umul24(g & 0xF0u, 0x204081u) & 0x10101010u);
+        hi = ((qs >> 4) & 0x0F0F0F0Fu) | (__umul24((g >> 16) & 0xF0u, 0x204081u) & 0x10101010u);
+        off = (_Float16)(-16.0f / 512.0f);
+    } else {
+        // kvalues_iq4nl (ggml-common.h:1110) + 128 as little-endian bytes
+        const uint32_t t0 = 0x3F2D1801u, t1 = 0x766A5D4Fu, t2 = 0xA6998D81u, t3 = 0xF1D9C5B5u;
+        const uint32_t sl = qs & 0x07070707u, sh = (qs >> 4) & 0x07070707u;
+        // byte j from the upper half of the table where its index has bit 3
+        uint32_t self = 0x03020100u;
+        asm("" : "+v"(self));                           // in a vector register: one v_and_or_b32 each
+        const uint32_t pl = ((qs >> 1) & 0x04040404u) | self, ph = ((qs >> 5) & 0x04040404u) | self;
+        lo = __builtin_amdgcn_perm(__builtin_amdgcn_perm(t3, t2, sl), __builtin_amdgcn_perm(t1, t0, sl), pl);
+        hi = __builtin_amdgcn_perm(__builtin_amdgcn_perm(t3, t2, sh), __builtin_amdgcn_perm(t1, t0, sh), ph);
+        off = (_Float16)(-128.0f / 512.0f);
+    }
+    const h2 mul = h2{(_Float16)32768.0f, (_Float16)32768.0f}, add = h2{off, off};
+    uint32_t h[4];
+    h[0] = h2bits(__builtin_elementwise_fma(as_h2(__builtin_amdgcn_perm(0u, lo, 0x0C020C00u)), mul, add));
+    h[1] = h2bits(__builtin_elementwise_fma(as_h2(__builtin_amdgcn_perm(0u, hi, 0x0C020C00u)), mul, add));
+    h[2] = h2bits(__builtin_elementwise_fma(as_h2(__builtin_amdgcn_perm(0u, lo, 0x0C030C01u)), mul, add));
+    h[3] = h2bits(__builtin_elementwise_fma(as_h2(__builtin_amdgcn_perm(0u, hi, 0x0C030C01u)), mul, add));
     h8 o;
     __builtin_memcpy(&o, h, 16);
     return o;
@@ -1348,186 +1378,192 @@ __device__ __forceinline__ void pf_down2_group(const PfParams & p, const PfTile 
     constexpr int NTOK = 16 * NT;
     static_assert(NTOK * 256 * CPS <= D2_XB, "a step's chunks fit an activation buffer");
     constexpr int BS = WT == T_Q5_0 ? 22 : 18;
-    constexpr int CW = BS / 2;                                  // dwords of a chunk (two blocks)
-    constexpr int NW = (4 * CW * CPS + 3 + 15) / 16;            // 16-byte loads of a step's row window
+    constexpr int SB = 2 * CPS * BS;                            // bytes of a row in a step
+    constexpr int G = ((14 + SB + 15) / 16) | 1;                // granules of a row's window (it starts on 16 bytes)
+    constexpr int NI = (32 * G + 63) / 64;                      // copies of a wave's windows
+    static_assert(NI * 1024 <= D2_WB, "a wave's windows fit");
     const int D = p.d_model, F = p.n_ff, NB = F / 32, NC = (NB + 1) / 2, NS = (NC + CPS - 1) / CPS;
     const int r0 = rb * PF_ROWS;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, l16 = lane & 15;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, l16 = lane & 15;
     const uint32_t rbytes = (uint32_t)(NB * BS);
     const uint8_t * W = tile.tier == 0 ? p.hot_dn + (uint64_t)tile.idx * p.hot_dn_stride
                                        : p.cold_dn + (uint64_t)tile.idx * p.cold_dn_stride;
-    // the slab as a buffer: a last chunk of one block (and a step's window)
-    // reads past its row (unused bytes; past the slab they read as zero)
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W), 0,
-                                                                         (int)((uint32_t)D * rbytes), 0x00020000);
-    if (tid < NTOK) L.pair[tid] = p.sorted[tile.begin + min(tid, tile.n - 1)];
+    const uint32_t last = (uint32_t)D * rbytes - 16u;           // the slab's last granule (slabs are whole granules)
+
+    // ---- copies.  Weights: granule g of row r of the wave, i = r G + g =
+    // 64 k + lane (past the rows: the last row's, into room that nothing
+    // reads).  d_model is a multiple of 256: every row exists.
+    uint32_t wrow[NI];
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+        const int i = min(64 * k + lane, 32 * G - 1), r = i / G, g = i - r * G;
+        wrow[k] = (uint32_t)(r0 + 32 * wave + r) * rbytes + 16u * (uint32_t)g;
+    }
+    auto copy_w = [&](int s) {
+        const uint8_t * w = W;
+        asm volatile("" : "+s"(w));
+#pragma unroll
+        for (int k = 0; k < NI; ++k)
+            lds_dma16(w + min((wrow[k] + (uint32_t)(SB * s)) & ~15u, last), L.w + 1024 * k);
+    };
+    copy_w(0);                                                  // before the pairs are known
+    if (tid < NTOK) {
+        const int pr = p.sorted[tile.begin + min(tid, tile.n - 1)];
+        L.pair[tid] = pr;
+        L.yoff[tid] = tid < tile.n ? (uint32_t)pr * (uint32_t)(4 * D) : 0x80000000u;
+    }
     __syncthreads();
 
-    // step s: chunks CPS s .. CPS s + CPS - 1, chunk c of the step at xb + c NTOK 256
-    auto copy_in = [&](int s, uint8_t * xb) {
-        const _Float16 * ah = p.ah;
-        const _Float16 * al = p.al;
-        asm volatile("" : "+s"(ah), "+s"(al));
-        // wave w moves pair blocks w NT + k (four pair slots each); a last
-        // chunk of one block reads its second block's slots from inside the row
+    // Activations: wave w moves pair blocks w NT + k (four pair slots each),
+    // chunk c of the step to xb + c NTOK 256; per lane the byte offset of its
+    // pair's row (high or low parts) and its 16 bytes' place
+    uint32_t arow[NT], apos[NT];
+    const uint32_t lo_off = (uint32_t)(reinterpret_cast<const uint8_t *>(p.al) - reinterpret_cast<const uint8_t *>(p.ah));
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+        const int j = 4 * (wave * NT + k) + (lane >> 4), sg = (lane & 15) ^ (j & 15);
+        arow[k] = (uint32_t)L.pair[j] * (uint32_t)(2 * F) + (sg < 8 ? 0u : lo_off);
+        apos[k] = 8u * (uint32_t)(sg & 7);
+    }
+    auto copy_act = [&](int s, uint8_t * xb) {
+        const uint8_t * ah = reinterpret_cast<const uint8_t *>(p.ah);
+        asm volatile("" : "+s"(ah));
 #pragma unroll
         for (int cc = 0; cc < CPS; ++cc) {
-            const int c = min(CPS * s + cc, NC - 1);
+            // a last chunk of one block reads its second block's slots from inside the row
+            const uint32_t c = (uint32_t)min(CPS * s + cc, NC - 1);
 #pragma unroll
-            for (int k = 0; k < NT; ++k) {
-                const int j = 4 * (wave * NT + k) + (lane >> 4);
-                const int sg = (lane & 15) ^ (j & 15);
-                const uint32_t off = (uint32_t)(L.pair[j] * F + min(64 * c + 8 * (sg & 7), F - 8));
-                lds_dma16((sg < 8 ? ah : al) + off, xb + NTOK * 256 * cc + 1024 * (wave * NT + k));
-            }
+            for (int k = 0; k < NT; ++k)
+                lds_dma16(ah + (arow[k] + 2u * min(64u * c + apos[k], (uint32_t)(F - 8))),
+                          xb + NTOK * 256 * cc + 1024 * (wave * NT + k));
         }
     };
+    // this lane's rows in the wave's windows, and where they start in the slab
     uint32_t voff[2];
 #pragma unroll
-    for (int rs = 0; rs < 2; ++rs) voff[rs] = (uint32_t)min(r0 + 32 * wave + 16 * rs + l16, D - 1) * rbytes;
-    // raw windows: from the dword at or below the step's start (a row of an
-    // odd block count starts 2 bytes into a dword), NW x 16 bytes
-    u32x4 wraw[2][NW];
-    uint32_t wsh[2];
-    auto load_rows = [&](int s) {
-#pragma unroll
-        for (int rs = 0; rs < 2; ++rs) {
-            const uint32_t st = voff[rs] + (uint32_t)(2 * BS * CPS * s);
-            const uint32_t v0 = st & ~3u;
-            wsh[rs] = 8u * (st & 3u);
-#pragma unroll
-            for (int k = 0; k < NW; ++k) wraw[rs][k] = __builtin_amdgcn_raw_buffer_load_b128(wr, v0 + 16 * k, 0, 0);
-        }
-    };
+    for (int rs = 0; rs < 2; ++rs) voff[rs] = (uint32_t)(r0 + 32 * wave + 16 * rs + l16) * rbytes;
 
     f4 y[2][NT];
 #pragma unroll
     for (int rs = 0; rs < 2; ++rs)
 #pragma unroll
         for (int ts = 0; ts < NT; ++ts) y[rs][ts] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t qrot = (4u * (uint32_t)q - 4u) & 31u;
 
-    auto step = [&](int s, const uint8_t * xb, uint8_t * xn) {
+    // one step; TAIL: the last one, whose blocks may run past n_ff
+    auto step = [&](int s, const uint8_t * xb, uint8_t * xn, auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        // this step's rows out of the registers the loads land in, the next
-        // step's copies and loads in flight during the MFMAs
-        DnWin wc[CPS][2];
+        if constexpr (!TAIL) copy_act(s + 1, xn);
+        DnRaw raw[2 * CPS][2];
+        uint32_t wsh[2];
 #pragma unroll
         for (int rs = 0; rs < 2; ++rs) {
-            uint32_t r[4 * NW];
+            const int at = (16 * rs + l16) * (16 * G) + (int)((voff[rs] + (uint32_t)(SB * s)) & 15u);
+            wsh[rs] = 8u * (uint32_t)(at & 2) ^ 16u;            // block b's shift: this, ^ 16 for odd b
 #pragma unroll
-            for (int k = 0; k < NW; ++k) {
-                r[4 * k] = wraw[rs][k].x;
-                r[4 * k + 1] = wraw[rs][k].y;
-                r[4 * k + 2] = wraw[rs][k].z;
-                r[4 * k + 3] = wraw[rs][k].w;
+            for (int b = 0; b < 2 * CPS; ++b) dn_raw_read<WT>(raw[b][rs], L.w, at + BS * b, q);
+        }
+        if constexpr (!TAIL) {
+            // the fields are in registers before the next windows land in their room
+#pragma unroll
+            for (int rs = 0; rs < 2; ++rs)
+#pragma unroll
+                for (int b = 0; b < 2 * CPS; ++b)
+                    dn_raw_here<WT>(raw[b][rs]);
+            copy_w(s + 1);
+        }
+        auto block = [&](int b) {
+            const uint8_t * xc = xb + NTOK * 256 * (b >> 1);
+            h8 bw[2];
+            float dw[2];
+#pragma unroll
+            for (int rs = 0; rs < 2; ++rs) {
+                bw[rs] = dn_frag<WT>(raw[b][rs], wsh[rs] ^ (16u * (b & 1)), qrot);
+                dw[rs] = h2f(raw[b][rs].d);
             }
 #pragma unroll
-            for (int cc = 0; cc < CPS; ++cc) {
-                uint32_t t[11];
+            for (int ts = 0; ts < NT; ++ts) {
+                const uint8_t * xr = xc + (16 * ts + l16) * 256;
+                h8 ah, al;
+                __builtin_memcpy(&ah, xr + 16 * ((4 * (b & 1) + q) ^ l16), 16);
+                __builtin_memcpy(&al, xr + 16 * ((8 + 4 * (b & 1) + q) ^ l16), 16);
 #pragma unroll
-                for (int i = 0; i < 11; ++i) {
-                    const int a = min(CW * cc + i, 4 * NW - 2);
-                    t[i] = __builtin_amdgcn_alignbit(r[a + 1], r[a], wsh[rs]);
+                for (int rs = 0; rs < 2; ++rs) {
+                    const f4 sb = mfma_f16(al, bw[rs], mfma_f16(ah, bw[rs], f4{0.0f, 0.0f, 0.0f, 0.0f}));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) y[rs][ts][r] = __builtin_fmaf(dw[rs], sb[r], y[rs][ts][r]);
                 }
-                wc[cc][rs].a = u32x4{t[0], t[1], t[2], t[3]};
-                wc[cc][rs].b = u32x4{t[4], t[5], t[6], t[7]};
-                wc[cc][rs].e = u32x3{t[8], t[9], t[10]};
             }
-        }
-        if (s + 1 < NS) {
-            copy_in(s + 1, xn);
-            load_rows(s + 1);
-        }
+        };
 #pragma unroll
-        for (int cc = 0; cc < CPS; ++cc) {
-            const int c = CPS * s + cc;
-            if (c < NC) {                                       // workgroup-uniform
-                const int cb = min(2, NB - 2 * c);
-                const uint8_t * xc = xb + NTOK * 256 * cc;
-                auto block = [&](auto bc) {
-                    constexpr int B = decltype(bc)::value;
-                    // B operand: lane (row l16, quarter q) holds values 8 q .. 8 q + 7 of block B
-                    h8 bw[2];
-                    float dw[2];
-#pragma unroll
-                    for (int rs = 0; rs < 2; ++rs) bw[rs] = down_frag_r<WT, B>(wc[cc][rs], q, dw[rs]);
-#pragma unroll
-                    for (int ts = 0; ts < NT; ++ts) {
-                        const uint8_t * xr = xc + (16 * ts + l16) * 256;
-                        h8 ah, al;
-                        __builtin_memcpy(&ah, xr + 16 * ((4 * B + q) ^ l16), 16);
-                        __builtin_memcpy(&al, xr + 16 * ((8 + 4 * B + q) ^ l16), 16);
-#pragma unroll
-                        for (int rs = 0; rs < 2; ++rs) {
-                            const f4 sb = mfma_f16(al, bw[rs], mfma_f16(ah, bw[rs], f4{0.0f, 0.0f, 0.0f, 0.0f}));
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) y[rs][ts][r] = __builtin_fmaf(dw[rs], sb[r], y[rs][ts][r]);
-                        }
-                    }
-                };
-                block(std::integral_constant<int, 0>{});
-                if (cb > 1) block(std::integral_constant<int, 1>{});
-            }
+        for (int b = 0; b < 2 * CPS; ++b) {
+            if (TAIL && 2 * CPS * s + b >= NB) break;           // workgroup-uniform
+            block(b);
         }
     };
 
-    copy_in(0, L.x0);
-    load_rows(0);
-    for (int s = 0; s < NS; s += 2) {
-        step(s, L.x0, L.x1);
-        if (s + 1 < NS) step(s + 1, L.x1, L.x0);
+    copy_act(0, L.x0);
+    int s = 0;
+    for (; s + 2 < NS; s += 2) {
+        step(s, L.x0, L.x1, std::false_type{});
+        step(s + 1, L.x1, L.x0, std::false_type{});
+    }
+    if (s + 1 < NS) {
+        step(s, L.x0, L.x1, std::false_type{});
+        step(s + 1, L.x1, L.x0, std::true_type{});
+    } else {
+        step(s, L.x0, L.x1, std::true_type{});
     }
     const float sc = tile.tier == 0 ? (p.s_hot ? p.s_hot[tile.idx] : 1.0f) : (p.s_cold ? p.s_cold[tile.idx] : 1.0f);
+    // buffer stores: a pair slot past the group holds an offset past the
+    // buffer, and its stores are dropped
+    const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
+        p.ydn, 0, (int)((uint32_t)p.T * (uint32_t)p.top_k * (uint32_t)(4 * D)), 0x00020000);
+    const uint32_t row4 = 4u * (uint32_t)(r0 + 32 * wave + l16);
 #pragma unroll
     for (int ts = 0; ts < NT; ++ts) {
+        const u32x4 off = *reinterpret_cast<const u32x4 *>(L.yoff + 16 * ts + 4 * q);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int j = 16 * ts + 4 * q + r;
-            if (j >= tile.n) continue;
-            float * out = p.ydn + (int64_t)L.pair[j] * D;
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int rs = 0; rs < 2; ++rs) {
-                const int row = r0 + 32 * wave + 16 * rs + l16;
-                if (row < D) out[row] = sc * y[rs][ts][r];
+                const float v = sc * (512.0f * y[rs][ts][r]);      // the weights were times 2^-9
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), yr, off[r] + row4 + 64u * rs, 0, 0);
             }
-        }
     }
 }
 
-// Grid: 8 x ceil(max_tiles / 8) x RB workgroups in one dimension, dealt to
-// the XCDs as the gate_up kernel's: all row blocks of a group on one XCD.
+// Grid (8, RB, ceil(max_tiles / 8)), dealt to the XCDs as the gate_up
+// kernel's: all row blocks of a group on one XCD.
 template <int HT, int CT>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_pf_down(const PfParams p) {
     __shared__ __align__(16) uint8_t x0[D2_XB];
     __shared__ __align__(16) uint8_t x1[D2_XB];
+    __shared__ __align__(16) uint8_t wb[(WG / 64) * D2_WB];
     __shared__ int pair[PF_TOK];
-    const Dn2Lds sm = {x0, x1, pair};
-    const int RB = (p.d_model + PF_ROWS - 1) / PF_ROWS;
-    const int i = blockIdx.x, k = i >> 3;
-    const int g = 8 * (k / RB) + (i & 7), rb = k - (k / RB) * RB;
+    __shared__ __align__(16) uint32_t yoff[PF_TOK];
+    const Dn2Lds sm = {x0, x1, wb + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * D2_WB, pair, yoff};
+    const int g = 8 * blockIdx.z + blockIdx.x, rb = blockIdx.y;
+    const PfTile tile = load_tile(p.tiles, p.max_tiles, g);
     if (g >= *p.n_tiles) return;
-    const PfTile tile = p.tiles[g];
     if (!tile_valid(p, tile) || tile.n <= 0 || tile.n > PF_TOK) return;
     const int nt = (tile.n + 15) >> 4;
-    static_assert(PF_TOK == 96, "six tile counts");
+    static_assert(PF_TOK == 64, "four tile counts");
     if ((tile.tier == 0 ? HT : CT) == T_Q5_0) {
         switch (nt) {
         case 1: pf_down2_group<T_Q5_0, 1, 2>(p, tile, sm, rb); break;
         case 2: pf_down2_group<T_Q5_0, 2, 2>(p, tile, sm, rb); break;
         case 3: pf_down2_group<T_Q5_0, 3, 1>(p, tile, sm, rb); break;
-        case 4: pf_down2_group<T_Q5_0, 4, 1>(p, tile, sm, rb); break;
-        case 5: pf_down2_group<T_Q5_0, 5, 1>(p, tile, sm, rb); break;
-        default: pf_down2_group<T_Q5_0, 6, 1>(p, tile, sm, rb); break;
+        default: pf_down2_group<T_Q5_0, 4, 1>(p, tile, sm, rb); break;
         }
     } else {
         switch (nt) {
         case 1: pf_down2_group<T_IQ4_NL, 1, 2>(p, tile, sm, rb); break;
         case 2: pf_down2_group<T_IQ4_NL, 2, 2>(p, tile, sm, rb); break;
         case 3: pf_down2_group<T_IQ4_NL, 3, 1>(p, tile, sm, rb); break;
-        case 4: pf_down2_group<T_IQ4_NL, 4, 1>(p, tile, sm, rb); break;
-        case 5: pf_down2_group<T_IQ4_NL, 5, 1>(p, tile, sm, rb); break;
-        default: pf_down2_group<T_IQ4_NL, 6, 1>(p, tile, sm, rb); break;
+        default: pf_down2_group<T_IQ4_NL, 4, 1>(p, tile, sm, rb); break;
         }
     }
 }
@@ -1547,7 +1583,7 @@ void launch_pf(F k, dim3 grid, hipStream_t s, hipEvent_t e0, hipEvent_t e1, cons
 }
 template <int HT, int CT>
 void launch_gu(int gelu, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const PfParams & p) {
-    const dim3 g2(8 * ((p.max_gtiles + 7) / 8) * ((p.n_ff + 63) / 64));
+    const dim3 g2(8, (p.n_ff + 63) / 64, (p.max_gtiles + 7) / 8);
     if (p.act_mode == AM_Q8_1) {
         if (gelu == SRC_GEGLU_TANH) launch_pf(k_pf_gate_up_q1<HT, CT, SRC_GEGLU_TANH>, g2, s, e0, e1, p);
         else launch_pf(k_pf_gate_up_q1<HT, CT, SRC_GEGLU_TABLE>, g2, s, e0, e1, p);
@@ -1588,7 +1624,7 @@ hipError_t launch_prefill(const PfParams & p0, int hgu, int cgu, int hdn, int cd
         if (err != hipSuccess) return err;
     }
     {
-        dim3 grid(8 * ((p.max_tiles + 7) / 8) * ((p.d_model + PF_ROWS - 1) / PF_ROWS));
+        dim3 grid(8, (p.d_model + PF_ROWS - 1) / PF_ROWS, (p.max_tiles + 7) / 8);
         if (hdn == T_Q5_0 && cdn == T_IQ4_NL) launch_pf(k_pf_down<T_Q5_0, T_IQ4_NL>, grid, s, e[2], e[3], p);
         else if (hdn == T_Q5_0 && cdn == T_Q5_0) launch_pf(k_pf_down<T_Q5_0, T_Q5_0>, grid, s, e[2], e[3], p);
         else if (hdn == T_IQ4_NL && cdn == T_IQ4_NL) launch_pf(k_pf_down<T_IQ4_NL, T_IQ4_NL>, grid, s, e[2], e[3], p);

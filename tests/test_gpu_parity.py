@@ -611,3 +611,25 @@ def test_prefill_in_a_workspace_of_a_shorter_call(gpu):
     torch.cuda.synchronize()
     for a, b in zip((out, ids, w), want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n_ff", [32, 64, 96, 224, 320])
+@pytest.mark.parametrize("T", [5, 150])
+@pytest.mark.parametrize("act_mode,gelu_mode", [(la.ACT_CPU, la.GELU_TABLE), (la.ACT_Q8_1, la.GELU_TANH)])
+def test_prefill_down_steps_and_groups(gpu, oracle, n_ff, T, act_mode, gelu_mode):
+    """The down GEMM at the edges of its K steps (one, two, an odd number of
+    32-blocks, rows that start 2 bytes into a dword, a last step past n_ff) and
+    of its groups (a few pairs per expert; 75 on average, so groups of every
+    tile count), hot and cold experts, the pools' last rows among them.  The
+    bars of check_flip_tolerant."""
+    torch = torch_mod()
+    spec = la.LayerSpec(d_model=256, n_ff=n_ff, n_expert=4, top_k=2)
+    say(f"prefill down n_ff={n_ff} T={T} act={act_mode}")
+    lay = layer(spec, 400 + n_ff, [0, 2], scales=True)
+    dl = la.DeviceLayer(lay, gpu, act_mode, gelu_mode)
+    x = tokens(401 + n_ff + T, T, spec.d_model)
+    xd = torch.from_numpy(x).to(gpu)
+    out, ids, w = (t.clone() for t in dl.forward(xd))
+    ref, _ = oracle.moe_experts(lay, x, ids.cpu().numpy(), w.cpu().numpy(), oracle_mode(act_mode, T), gelu_mode)
+    assert np.isfinite(out.cpu().numpy()).all()
+    check_flip_tolerant(out.cpu().numpy(), ref)
