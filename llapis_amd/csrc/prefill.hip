@@ -16,9 +16,8 @@
 //                  (both exact in fp16) for the Q4_K mins term
 //                  (pf_quant_x1: q8_1, as exact fp16 parts).
 //   k_pf_gate_up   grouped GEMM per (group, 64 gate rows + the 64 matching up
-//                  rows), on groups of its own (<= 48 pairs of a Q4_K expert,
-//                  <= 64 of an IQ2_S one), the full groups first, every row
-//                  block of a group on one XCD.  Each super-block of weights
+//                  rows), on groups of its own (<= 48 pairs), the full groups
+//                  first, every row block of a group on one XCD.  Each super-block of weights
 //                  is expanded once into int8 MFMA operands and used for
 //                  every token of the group.  The sub-block scales are folded
 //                  into the weights: Q4_K's 6-bit scale splits as 8 sh + sl,
@@ -428,38 +427,42 @@ __device__ __forceinline__ void q8_store32(float v, _Float16 * hi, _Float16 * lo
 // One workgroup per (gate_up group, 64 gate rows + the 64 matching up rows).
 // Wave w owns local rows 32 w .. 32 w + 31 (waves 0, 1: gate rows; 2, 3: the
 // up rows of the same indices) as two 16-row MFMA tiles.  The load unit
-// copies the group's activations of the next super-block (and the Q4_K rows)
-// into LDS (global_load_lds) while the current one is expanded and used;
-// IQ2_S rows go straight to registers with buffer loads, as their 82-byte
-// super-blocks are not 16-byte aligned.  Two buffers of each kind, so one
-// barrier per super-block both publishes super-block s and retires s - 1.
-// A token's 16-byte chunk c of a super-block sits in slot c ^ (token & 15)
-// of its 256-byte LDS row: the 16 tokens of an MFMA fragment read 16
-// distinct slots, so the fragment loads meet no bank conflict.
+// copies the group's activations of the next super-block into LDS
+// (global_load_lds) while the current one is expanded and used: two buffers,
+// so one barrier per super-block both publishes super-block s and retires
+// s - 1.  A wave's Q4_K rows come the same way into room of its own: it takes
+// a super-block's fields into registers and then starts the next one's copy
+// into the same room, so one buffer is enough and three workgroups share a CU
+// instead of two (the kernel is bound by VALU issue and, between a
+// workgroup's steps, by waits that other workgroups fill: fastest traced
+// dispatches 126 -> 110 us at 512 tokens, dual K = 57, 283 -> 236 us at 1900
+// tokens, all hot, 40 -> 36 us at 12 tokens).  IQ2_S rows go straight to registers with buffer loads, as their
+// 82-byte super-blocks are not 16-byte aligned.  A token's 16-byte chunk c of
+// a super-block sits in slot c ^ (token & 15) of its 256-byte LDS row: the 16
+// tokens of an MFMA fragment read 16 distinct slots, so the fragment loads
+// meet no bank conflict.
 
-constexpr int G2_TOKQ4 = 48;            // pairs per group of a Q4_K expert (at 64 the kernel spills registers)
-constexpr int G2_TOKIQ2 = 64;           // of an IQ2_S expert (its tables share the LDS)
-static_assert(G2_TOKQ4 <= PF_GTOK && G2_TOKIQ2 <= PF_GTOK, "group caps");
-constexpr int G2_TOKMAX = G2_TOKQ4 > G2_TOKIQ2 ? G2_TOKQ4 : G2_TOKIQ2;
-constexpr int G2_MBT = (G2_TOKQ4 + 31) / 32 * 32;     // tokens of a mins buffer: 32 per moving wave
+constexpr int G2_TOK = 48;              // pairs per group (three 16-token MFMA tiles)
+static_assert(G2_TOK <= PF_GTOK, "group cap");
+constexpr int G2_MBT = (G2_TOK + 31) / 32 * 32;       // tokens of a mins buffer: 32 per moving wave
 
 // LDS of one workgroup.  Each of the two buffers of a kind is a separate
 // object: the compiler then knows that a copy into one does not write the
 // other, and it does not make reads of the current buffer wait for the copy
 // of the next.  The epilogue stages gate rows in x0 and up rows in x1
-// ([64 rows][NTOK + 1] floats each); the IQ2_S tables live in w0 / w1 (that
-// format's rows go straight to registers).
-constexpr int G2_XB = 64 * (G2_TOKMAX + 1) * 4;
-constexpr int G2_WB = PF_ROWS * 144;                      // one super-block of 128 Q4_K rows
-static_assert(G2_XB >= G2_TOKQ4 * 256 && G2_XB >= G2_TOKIQ2 * 256, "activation buffers");
-static_assert(G2_WB >= 1024 * 8 && G2_WB >= 16 * 16, "IQ2_S tables fit the weight buffers");
+// ([64 rows][NTOK + 1] floats each); the IQ2_S tables live in the Q4_K rows'
+// room.
+constexpr int G2_XB = 64 * (G2_TOK + 1) * 4;
+constexpr int G2_WROW = 5 * 1024;                         // a wave's 32 Q4_K super-block rows (4.5 copies)
+static_assert(G2_XB >= G2_TOK * 256, "activation buffers");
+static_assert(32 * 144 <= G2_WROW && 4 * G2_WROW >= 1024 * 8 + 16 * 16, "rows, IQ2_S tables");
 struct Gu2Lds {
     uint8_t * x0; uint8_t * x1;                   // the group's q8_K values of one super-block
-    uint8_t * w0; uint8_t * w1;                   // Q4_K: the 128 rows of one super-block, [row][144]
+    uint8_t * w;                                  // Q4_K: this wave's 32 rows of one super-block, [row][144]
     _Float16 * mb0; _Float16 * mb1;               // their per-32 sums (32 hi + lo), Q4_K
     float * d80; float * d81;                     // their q8_K scales
-    uint2 * codes;                                // IQ2_S grid: a level code per value (in w0)
-    u32x4 * split;                                // Iq2sSplit (in w1)
+    uint2 * codes;                                // IQ2_S grid: a level code per value
+    u32x4 * split;                                // Iq2sSplit
     int * tok; int * pair;
 };
 
@@ -522,16 +525,36 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
     constexpr bool Q4 = WT == T_Q4_K;
     static_assert(Q4 || WT == T_IQ2_S, "gate_up formats");
     constexpr int NTOK = 16 * NT;
-    static_assert(NTOK <= (Q4 ? G2_TOKQ4 : G2_TOKIQ2), "group fits the LDS");
+    static_assert(NTOK <= G2_TOK, "group fits the LDS");
     constexpr int BB = Q4 ? 144 : 82;                           // bytes per super-block
     const int F = p.n_ff, NSB = p.d_model / 256, K = p.top_k, D = p.d_model;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, l16 = lane & 15;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, l16 = lane & 15;
     const uint32_t rbytes = (uint32_t)(NSB * BB);
     const uint8_t * W = tile.tier == 0 ? p.hot_gu + (uint64_t)tile.idx * p.hot_gu_stride
                                        : p.cold_gu + (uint64_t)tile.idx * p.cold_gu_stride;
     const uint32_t slab = (uint32_t)(2u * (uint32_t)F * rbytes);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W), 0, (int)slab,
                                                                          0x00020000);
+    // a wave's Q4_K rows: granule i = 64 k + lane is chunk i mod 9 of its row
+    // i / 9 (past the rows: the last one's, into room that nothing reads)
+    uint32_t wrow[Q4 ? 5 : 1];
+    if constexpr (Q4) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const int i = min(64 * k + lane, 32 * 9 - 1), r = i / 9, c = i - 9 * r;
+            const int gi = min(64 * rb + 32 * (wave & 1) + r, F - 1);
+            wrow[k] = (uint32_t)(wave < 2 ? gi : F + gi) * rbytes + 16u * (uint32_t)c;
+        }
+    }
+    auto copy_w = [&](int s) {
+        if constexpr (Q4) {
+            const uint8_t * wsb = W + 144 * s;
+            asm volatile("" : "+s"(wsb));
+#pragma unroll
+            for (int k = 0; k < 5; ++k) lds_dma16(wsb + wrow[k], L.w + 1024 * k);
+        }
+    };
+    copy_w(0);                                                  // before the pairs are known
     if (tid < NTOK) {
         const int qp = p.sorted[tile.begin + min(tid, tile.n - 1)];
         L.pair[tid] = qp;
@@ -552,23 +575,7 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
     // lanes a token, lane slot i ^ token), the mins sums of 32 tokens (wave <
     // ceil(NT / 2), Q4_K) and the scales of 64 tokens (wave < ceil(NT / 4))
     const bool mb_mover = Q4 && 32 * wave < NTOK, d8_mover = 64 * wave < NTOK;
-    // Q4_K rows: 128 rows x 9 chunks of one super-block, [row][144] in LDS;
-    // copy j (0..17, wave w takes j = w, w + 4, ...) moves chunks 64 j .. + 63
-    auto wrow_off = [&](int j) {
-        const int i = 64 * j + lane, r = i / 9, c = i - 9 * r;
-        const int gi = min(64 * rb + (r & 63), F - 1);
-        return (uint32_t)(r < 64 ? gi : F + gi) * rbytes + 16u * (uint32_t)c;
-    };
-    auto copy_in = [&](int s, uint8_t * xb, _Float16 * mbb, float * d8b, uint8_t * wb) {
-        if constexpr (Q4) {
-            const uint8_t * wsb = W + 144 * s;
-            asm volatile("" : "+s"(wsb));
-#pragma unroll
-            for (int k = 0; k < 5; ++k) {
-                const int j = wave + 4 * k;
-                if (j < 18) lds_dma16(wsb + wrow_off(j), wb + 1024 * j);
-            }
-        }
+    auto copy_in = [&](int s, uint8_t * xb, _Float16 * mbb, float * d8b) {
         // the super-block's offsets are made opaque, so that the compiler
         // keeps one uniform base per copy (an SGPR pair) and the lanes' 32-bit
         // offsets (recomputed from the token list: no registers held)
@@ -615,13 +622,12 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
 #pragma unroll
         for (int ts = 0; ts < NT; ++ts) y[rs][ts] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     // per-lane constants of the Q4_K expansion: the byte of this lane's
-    // sub-block scale in both 16-bit halves (sub-block 2 st + q / 2: byte
-    // q / 2 for even st, 2 + q / 2 for odd), the nibble, and the mins
+    // sub-block scale in both 16-bit halves (sub-blocks 4 u + 2 (q / 2) for the
+    // low nibbles and the one after it for the high ones), and the mins
     // operand's (1024 + m) * mult + off (32 m, m or 0 by quarter)
-    const uint32_t jb_e = (uint32_t)(q >> 1), jb_o = 2u + (uint32_t)(q >> 1);
+    const uint32_t jb_e = 2u * (uint32_t)(q >> 1), jb_o = jb_e + 1u;
     const uint32_t sel_even = jb_e | 0x0C00u | (jb_e << 16) | 0x0C000000u;
     const uint32_t sel_odd = jb_o | 0x0C00u | (jb_o << 16) | 0x0C000000u;
-    const uint32_t nib_shift = 4u * (uint32_t)(q >> 1);
     const _Float16 mm = q == 0 ? (_Float16)32.0f : q == 1 ? (_Float16)1.0f : (_Float16)0.0f;
     const _Float16 mo = q == 0 ? (_Float16)(-32768.0f) : q == 1 ? (_Float16)(-1024.0f) : (_Float16)0.0f;
     const h2 mn_mul = h2{mm, mm}, mn_off = h2{mo, mo};
@@ -633,16 +639,21 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
     // into int32 accumulators that live across the slices -- so one slice's
     // expansion (VALU) overlaps the previous slice's MFMAs -- and last the
     // per-output scaling of every tile.
-    auto step = [&](int s, const uint8_t * xb, const _Float16 * mbb, const float * d8b, const uint8_t * wb,
-                    uint8_t * xn, _Float16 * mbn, float * d8n, uint8_t * wn) {
+    auto step = [&](int s, const uint8_t * xb, const _Float16 * mbb, const float * d8b,
+                    uint8_t * xn, _Float16 * mbn, float * d8n, auto more) {
+        constexpr bool MORE = decltype(more)::value;            // a super-block follows
         // this wave's copies and rows of super-block s have landed; after the
         // barrier every wave's have, and every wave is done with s - 1
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
 
-        // ---- per row tile: Q4_K lane (row l16, quarter q) takes values 64 st
-        // + 16 q of slice st (sub-block 2 st + q / 2); IQ2_S the 16-value group
-        // 4 q + st.  The activations are read in the same order.  The
+        if constexpr (MORE) copy_in(s + 1, xn, mbn, d8n);
+
+        // ---- per row tile: Q4_K lane (row l16, quarter q) takes the 16 bytes
+        // 64 u + 16 q of the nibbles, u = 0, 1: the low ones are its slice 2 u
+        // (sub-block 4 u + 2 (q / 2), half q & 1), the high ones slice 2 u + 1
+        // (the sub-block after it); IQ2_S the 16-value group 4 q + st.  The
+        // activations are read in the same order.  The
         // sub-block scales are folded in: Q4_K's 6-bit scale as 8 sh + sl
         // (q sh, q sl <= 105), IQ2_S's grid (2 ls + 1) as 64 h + l.
         float dr[2], mr[2];
@@ -650,11 +661,26 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
         uint2 qs8[2], sg8[2];                                // IQ2_S
         uint32_t qh2[2], sc2[2];
         h8 bm[2];
+        u32x4 hdr4[Q4 ? 2 : 1], nib[Q4 ? 2 : 1][2];
+        if constexpr (Q4) {
+#pragma unroll
+            for (int rs = 0; rs < 2; ++rs) {
+                const uint8_t * wrw = L.w + (16 * rs + l16) * 144;
+                hdr4[rs] = *reinterpret_cast<const u32x4 *>(wrw);
+                nib[rs][0] = *reinterpret_cast<const u32x4 *>(wrw + 16 + 16 * q);
+                nib[rs][1] = *reinterpret_cast<const u32x4 *>(wrw + 80 + 16 * q);
+            }
+            if constexpr (MORE) {
+                // in registers before the next super-block lands in their room
+#pragma unroll
+                for (int rs = 0; rs < 2; ++rs) asm volatile("" : "+v"(hdr4[rs]), "+v"(nib[rs][0]), "+v"(nib[rs][1]));
+                copy_w(s + 1);
+            }
+        }
 #pragma unroll
         for (int rs = 0; rs < 2; ++rs) {
             if constexpr (Q4) {
-                const uint8_t * wrw = wb + (32 * wave + 16 * rs + l16) * 144;
-                const u32x4 hdr = *reinterpret_cast<const u32x4 *>(wrw);
+                const u32x4 hdr = hdr4[rs];
                 dr[rs] = h2f(hdr.x & 0xFFFF);
                 mr[rs] = h2f(hdr.x >> 16);
                 // 6-bit scales and mins, four per dword (get_scale_min_k4,
@@ -691,16 +717,19 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
             }
         }
 
-        // ---- the next super-block in flight during this one's MFMAs
-        if (s + 1 < NSB) {
-            copy_in(s + 1, xn, mbn, d8n, wn);
-            load_rows(s + 1);
-        }
+        // ---- the next super-block's IQ2_S rows in flight during this one's MFMAs
+        if constexpr (MORE) load_rows(s + 1);
 
-        // ---- slice by slice: expand, then every tile's MFMAs
+        // ---- slice by slice: expand, then every tile's MFMAs; a three-tile
+        // group takes its row tiles one after the other (with the accumulators
+        // of both, 168 registers -- three waves a SIMD -- spill)
+        constexpr int RG = NT >= 3 ? 1 : 2;
+#pragma unroll
+        for (int rg = 0; rg < 2; rg += RG) {
+        if (RG == 1) asm volatile("" ::: "memory");             // fragments are read again, not kept
         v4i ah[2][NT], al[2][NT];
 #pragma unroll
-        for (int rs = 0; rs < 2; ++rs)
+        for (int rs = rg; rs < rg + RG; ++rs)
 #pragma unroll
             for (int ts = 0; ts < NT; ++ts) {
                 ah[rs][ts] = v4i{0, 0, 0, 0};
@@ -710,17 +739,16 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
         for (int st = 0; st < 4; ++st) {
             v4i bh[2], bl[2];
 #pragma unroll
-            for (int rs = 0; rs < 2; ++rs) {
+            for (int rs = rg; rs < rg + RG; ++rs) {
                 if constexpr (Q4) {
-                    const uint8_t * wrw = wb + (32 * wave + 16 * rs + l16) * 144;
-                    const u32x4 v = *reinterpret_cast<const u32x4 *>(wrw + 16 + 32 * st + 16 * (q & 1));
+                    const u32x4 v = nib[rs][st >> 1];
                     const uint32_t sel = (st & 1) ? sel_odd : sel_even;
                     const uint32_t sh2 = __builtin_amdgcn_perm(0u, st < 2 ? sh03[rs] : sh47[rs], sel);
                     const uint32_t sl2 = __builtin_amdgcn_perm(0u, st < 2 ? sl03[rs] : sl47[rs], sel);
                     const uint32_t w4v[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const uint32_t nb = (w4v[i] >> nib_shift) & 0x0F0F0F0Fu;
+                        const uint32_t nb = ((st & 1) ? w4v[i] >> 4 : w4v[i]) & 0x0F0F0F0Fu;
                         bh[rs][i] = (int)bytes_mul(nb, sh2);
                         bl[rs][i] = (int)bytes_mul(nb, sl2);
                     }
@@ -743,10 +771,10 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
 #pragma unroll
             for (int ts = 0; ts < NT; ++ts) {
                 const uint8_t * xr = xb + (16 * ts + l16) * 256;
-                const int c = Q4 ? q + 4 * st : 4 * q + st;
+                const int c = Q4 ? 8 * (st >> 1) + 4 * (q >> 1) + 2 * (st & 1) + (q & 1) : 4 * q + st;
                 const v4i a = as_v4i(*reinterpret_cast<const u32x4 *>(xr + 16 * (c ^ l16)));
 #pragma unroll
-                for (int rs = 0; rs < 2; ++rs) {
+                for (int rs = rg; rs < rg + RG; ++rs) {
                     ah[rs][ts] = mfma_i8(a, bh[rs], ah[rs][ts]);
                     al[rs][ts] = mfma_i8(a, bl[rs], al[rs][ts]);
                 }
@@ -769,7 +797,7 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
                 __builtin_memcpy(&am, &mv, 16);
             }
 #pragma unroll
-            for (int rs = 0; rs < 2; ++rs) {
+            for (int rs = rg; rs < rg + RG; ++rs) {
                 if constexpr (Q4) {
                     const f4 m = mfma_f16(am, bm[rs], f4{0.0f, 0.0f, 0.0f, 0.0f});
 #pragma unroll
@@ -787,13 +815,25 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
                 }
             }
         }
+        if constexpr (RG == 1) {                                // the sums are done here, not in the next step
+#pragma unroll
+            for (int ts = 0; ts < NT; ++ts) asm volatile("" : "+v"(y[rg][ts]));
+        }
+        }
     };
 
-    copy_in(0, L.x0, L.mb0, L.d80, L.w0);
+    copy_in(0, L.x0, L.mb0, L.d80);
     load_rows(0);
-    for (int s = 0; s < NSB; s += 2) {
-        step(s, L.x0, L.mb0, L.d80, L.w0, L.x1, L.mb1, L.d81, L.w1);
-        if (s + 1 < NSB) step(s + 1, L.x1, L.mb1, L.d81, L.w1, L.x0, L.mb0, L.d80, L.w0);
+    int s = 0;
+    for (; s + 2 < NSB; s += 2) {
+        step(s, L.x0, L.mb0, L.d80, L.x1, L.mb1, L.d81, std::true_type{});
+        step(s + 1, L.x1, L.mb1, L.d81, L.x0, L.mb0, L.d80, std::true_type{});
+    }
+    if (s + 1 < NSB) {
+        step(s, L.x0, L.mb0, L.d80, L.x1, L.mb1, L.d81, std::true_type{});
+        step(s + 1, L.x1, L.mb1, L.d81, L.x0, L.mb0, L.d80, std::false_type{});
+    } else {
+        step(s, L.x0, L.mb0, L.d80, L.x1, L.mb1, L.d81, std::false_type{});
     }
 
     // ---- epilogue: every tile's outputs into LDS at once (gate rows in x0,
@@ -847,39 +887,36 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
 // group 8 z + x, row block y: all row blocks of a group run on XCD x and read
 // its activations through one L2, and every XCD takes the full groups first.
 template <int HT, int CT, int GSRC>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_pf_gate_up(const PfParams p) {
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_pf_gate_up(const PfParams p) {
     __shared__ __align__(16) uint8_t x0[G2_XB];
     __shared__ __align__(16) uint8_t x1[G2_XB];
     __shared__ __align__(16) _Float16 mb0[G2_MBT * 16];
     __shared__ __align__(16) _Float16 mb1[G2_MBT * 16];
     __shared__ __align__(16) float d80[128];
     __shared__ __align__(16) float d81[128];
-    __shared__ __align__(16) uint8_t w0[G2_WB];
-    __shared__ __align__(16) uint8_t w1[G2_WB];
-    __shared__ int tok[G2_TOKMAX], pair[G2_TOKMAX];
-    const Gu2Lds sm = {x0, x1, w0, w1, mb0, mb1, d80, d81, reinterpret_cast<uint2 *>(w0),
-                       reinterpret_cast<u32x4 *>(w1), tok, pair};
+    __shared__ __align__(16) uint8_t w[(WG / 64) * G2_WROW];
+    __shared__ int tok[G2_TOK], pair[G2_TOK];
+    const Gu2Lds sm = {x0, x1, w + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * G2_WROW, mb0, mb1, d80, d81,
+                       reinterpret_cast<uint2 *>(w), reinterpret_cast<u32x4 *>(w + 1024 * 8), tok, pair};
     const int g = 8 * blockIdx.z + blockIdx.x, rb = blockIdx.y;
     const PfTile tile = load_tile(p.gtiles, p.max_gtiles, g);
     if (g >= *p.n_gtiles) return;
     if (!tile_valid(p, tile) || tile.n <= 0) return;
     const int wt = tile.tier == 0 ? HT : CT;
     const int nt = (tile.n + 15) >> 4;
+    if (tile.n > G2_TOK) return;
+    static_assert(G2_TOK == 48, "three tile counts");
     if (wt == T_Q4_K) {
-        if (tile.n > G2_TOKQ4) return;
         switch (nt) {
         case 1: pf_gu2_group<T_Q4_K, GSRC, 1>(p, tile, sm, rb); break;
         case 2: pf_gu2_group<T_Q4_K, GSRC, 2>(p, tile, sm, rb); break;
-        case 3: pf_gu2_group<T_Q4_K, GSRC, 3>(p, tile, sm, rb); break;
         default: pf_gu2_group<T_Q4_K, GSRC, 3>(p, tile, sm, rb); break;
         }
     } else {
-        if (tile.n > G2_TOKIQ2) return;
         switch (nt) {
         case 1: pf_gu2_group<T_IQ2_S, GSRC, 1>(p, tile, sm, rb); break;
         case 2: pf_gu2_group<T_IQ2_S, GSRC, 2>(p, tile, sm, rb); break;
-        case 3: pf_gu2_group<T_IQ2_S, GSRC, 3>(p, tile, sm, rb); break;
-        default: pf_gu2_group<T_IQ2_S, GSRC, 4>(p, tile, sm, rb); break;
+        default: pf_gu2_group<T_IQ2_S, GSRC, 3>(p, tile, sm, rb); break;
         }
     }
 }
@@ -1592,9 +1629,8 @@ void launch_gu(int gelu, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const PfPa
         else launch_pf(k_pf_gate_up<HT, CT, SRC_GEGLU_TABLE>, g2, s, e0, e1, p);
     }
 }
-// pairs per gate_up group of an expert in format t (the Q4_K kernel holds
-// 128 tokens' activations in LDS; IQ2_S's tables take the room of half)
-int gate_up_cap(int t) { return t == T_Q4_K ? G2_TOKQ4 : G2_TOKIQ2; }
+// pairs per gate_up group of an expert in format t
+int gate_up_cap(int) { return G2_TOK; }
 // in the q8_1 mode (1 KB of activation parts per token and super-block)
 int gate_up_cap_q1(int t) { return t == T_Q4_K ? PF_TOK1Q4 : PF_TOK1IQ2; }
 }  // namespace

@@ -633,3 +633,20 @@ def test_prefill_down_steps_and_groups(gpu, oracle, n_ff, T, act_mode, gelu_mode
     ref, _ = oracle.moe_experts(lay, x, ids.cpu().numpy(), w.cpu().numpy(), oracle_mode(act_mode, T), gelu_mode)
     assert np.isfinite(out.cpu().numpy()).all()
     check_flip_tolerant(out.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("d_model", [256, 512, 768, 1280])
+@pytest.mark.parametrize("T", [7, 100])
+def test_prefill_gate_up_super_blocks(gpu, oracle, d_model, T):
+    """The gate_up GEMM over one, two, an odd number and more super-blocks (its
+    K loop is peeled by parity), groups of one to three tiles, the last row
+    block half empty (n_ff 96).  The bars of check_flip_tolerant."""
+    torch = torch_mod()
+    spec = la.LayerSpec(d_model=d_model, n_ff=96, n_expert=6, top_k=2)
+    say(f"prefill gate_up d_model={d_model} T={T}")
+    lay = layer(spec, 500 + d_model, [1, 3, 5])
+    dl = la.DeviceLayer(lay, gpu)
+    x = tokens(501 + d_model + T, T, d_model)
+    out, ids, w = dl.forward(torch.from_numpy(x).to(gpu))
+    ref, _ = oracle.moe_experts(lay, x, ids.cpu().numpy(), w.cpu().numpy())
+    check_flip_tolerant(out.cpu().numpy(), ref)
