@@ -489,7 +489,10 @@ int router_parts_floats(int T, int E) { return RSPLIT * T * E; }
 hipError_t launch_router_mfma(const float * x, int T, const float * w_r, int d, int E, float * parts, hipStream_t s) {
     if (d % (16 * RSPLIT) != 0 || T <= 0 || E <= 0) return hipErrorInvalidValue;
     dim3 grid((T + RT - 1) / RT, (E + RT - 1) / RT, RSPLIT);
-    if (d / RSPLIT <= RKC_MAX)
+    // the staged kernel's 100 KB leave room for one workgroup a CU: ahead where
+    // every workgroup finds one (256: 9.0 against 9.5 us), behind where they
+    // queue (960, 1900 tokens: 30 against 21 us)
+    if (d / RSPLIT <= RKC_MAX && grid.x * grid.y * grid.z <= 256)
         hipLaunchKernelGGL(k_router_mfma_st, grid, dim3(WG), 0, s, x, T, w_r, d, E, d / RSPLIT, parts);
     else hipLaunchKernelGGL(k_router_mfma, grid, dim3(WG), 0, s, x, T, w_r, d, E, d / RSPLIT, parts);
     return hipGetLastError();

@@ -650,3 +650,18 @@ def test_prefill_gate_up_super_blocks(gpu, oracle, d_model, T):
     out, ids, w = dl.forward(torch.from_numpy(x).to(gpu))
     ref, _ = oracle.moe_experts(lay, x, ids.cpu().numpy(), w.cpu().numpy())
     check_flip_tolerant(out.cpu().numpy(), ref)
+
+
+def test_prefill_router_of_a_long_call(gpu):
+    """The router of a call with more workgroups than CUs takes the slice by
+    slice kernel, shorter calls the staged one: the same sums, so the same ids
+    and weights bit for bit as the call's 256-token pieces."""
+    torch = torch_mod()
+    spec = SMALL
+    say("prefill router T=1100")
+    dl = la.DeviceLayer(_layer_case(spec, 91, 6, True), gpu)
+    x = torch.from_numpy(tokens(602, 1100, spec.d_model)).to(gpu)
+    _, ids, w = (t.clone() for t in dl.forward(x))
+    for t0 in range(0, 1100, 256):
+        _, i, v = dl.forward(x[t0:t0 + 256].contiguous())
+        assert torch.equal(i, ids[t0:t0 + 256]) and torch.equal(v, w[t0:t0 + 256]), t0
