@@ -430,15 +430,16 @@ __device__ __forceinline__ void q8_store32(float v, _Float16 * hi, _Float16 * lo
 // copies the group's activations of the next super-block into LDS
 // (global_load_lds) while the current one is expanded and used: two buffers,
 // so one barrier per super-block both publishes super-block s and retires
-// s - 1.  A wave's Q4_K rows come the same way into room of its own: it takes
+// s - 1.  A wave's rows come the same way into room of its own: it takes
 // a super-block's fields into registers and then starts the next one's copy
 // into the same room, so one buffer is enough and three workgroups share a CU
 // instead of two (the kernel is bound by VALU issue and, between a
 // workgroup's steps, by waits that other workgroups fill: fastest traced
 // dispatches 126 -> 110 us at 512 tokens, dual K = 57, 283 -> 236 us at 1900
-// tokens, all hot, 40 -> 36 us at 12 tokens).  IQ2_S rows go straight to registers with buffer loads, as their
-// 82-byte super-blocks are not 16-byte aligned.  A token's 16-byte chunk c of
-// a super-block sits in slot c ^ (token & 15) of its 256-byte LDS row: the 16
+// tokens, all hot, 40 -> 36 us at 12 tokens).  IQ2_S rows, read straight into
+// registers before, came in 64 accesses of the L1 a 12-byte load: through the
+// windows 110 -> 105 us at 512 tokens, 36 -> 32 us at 12.  A token's 16-byte chunk c of a
+// super-block sits in slot c ^ (token & 15) of its 256-byte LDS row: the 16
 // tokens of an MFMA fragment read 16 distinct slots, so the fragment loads
 // meet no bank conflict.
 
@@ -455,10 +456,15 @@ constexpr int G2_MBT = (G2_TOK + 31) / 32 * 32;       // tokens of a mins buffer
 constexpr int G2_XB = 64 * (G2_TOK + 1) * 4;
 constexpr int G2_WROW = 5 * 1024;                         // a wave's 32 Q4_K super-block rows (4.5 copies)
 static_assert(G2_XB >= G2_TOK * 256, "activation buffers");
-static_assert(32 * 144 <= G2_WROW && 4 * G2_WROW >= 1024 * 8 + 16 * 16, "rows, IQ2_S tables");
+// IQ2_S: a wave's 32 rows' windows of a super-block, six granules each (the
+// window starts on 16 bytes: 14 + 82 bytes at most).  The rows' room is two
+// objects: Q4_K waves 0, 1 and 2, 3; IQ2_S the windows and the tables.
+constexpr int G2_IQROW = 3 * 1024;
+constexpr int G2_WA = 4 * G2_IQROW, G2_WB = 2 * G2_WROW;
+static_assert(32 * 144 <= G2_WROW && 2 * G2_WROW <= G2_WA && 1024 * 8 + 16 * 16 <= G2_WB, "rows and tables fit");
 struct Gu2Lds {
     uint8_t * x0; uint8_t * x1;                   // the group's q8_K values of one super-block
-    uint8_t * w;                                  // Q4_K: this wave's 32 rows of one super-block, [row][144]
+    uint8_t * w;                                  // this wave's 32 rows of one super-block: Q4_K [row][144], IQ2_S [row][96]
     _Float16 * mb0; _Float16 * mb1;               // their per-32 sums (32 hi + lo), Q4_K
     float * d80; float * d81;                     // their q8_K scales
     uint2 * codes;                                // IQ2_S grid: a level code per value
@@ -532,26 +538,25 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
     const uint32_t rbytes = (uint32_t)(NSB * BB);
     const uint8_t * W = tile.tier == 0 ? p.hot_gu + (uint64_t)tile.idx * p.hot_gu_stride
                                        : p.cold_gu + (uint64_t)tile.idx * p.cold_gu_stride;
-    const uint32_t slab = (uint32_t)(2u * (uint32_t)F * rbytes);
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W), 0, (int)slab,
-                                                                         0x00020000);
-    // a wave's Q4_K rows: granule i = 64 k + lane is chunk i mod 9 of its row
-    // i / 9 (past the rows: the last one's, into room that nothing reads)
-    uint32_t wrow[Q4 ? 5 : 1];
-    if constexpr (Q4) {
+    const uint32_t last = 2u * (uint32_t)F * rbytes - 16u;      // the slab's last granule (slabs are whole granules)
+    // a wave's rows of a super-block: Q4_K: granule i = 64 k + lane is chunk
+    // i mod 9 of its row i / 9 (past the rows: the last one's, into room that
+    // nothing reads); IQ2_S: granule i mod 6 of the window of row i / 6
+    constexpr int RG16 = Q4 ? 9 : 6, NCW = Q4 ? 5 : 3;
+    uint32_t wrow[NCW];
 #pragma unroll
-        for (int k = 0; k < 5; ++k) {
-            const int i = min(64 * k + lane, 32 * 9 - 1), r = i / 9, c = i - 9 * r;
-            const int gi = min(64 * rb + 32 * (wave & 1) + r, F - 1);
-            wrow[k] = (uint32_t)(wave < 2 ? gi : F + gi) * rbytes + 16u * (uint32_t)c;
-        }
+    for (int k = 0; k < NCW; ++k) {
+        const int i = min(64 * k + lane, 32 * RG16 - 1), r = i / RG16, c = i - RG16 * r;
+        const int gi = min(64 * rb + 32 * (wave & 1) + r, F - 1);
+        wrow[k] = (uint32_t)(wave < 2 ? gi : F + gi) * rbytes + 16u * (uint32_t)c;
     }
     auto copy_w = [&](int s) {
-        if constexpr (Q4) {
-            const uint8_t * wsb = W + 144 * s;
-            asm volatile("" : "+s"(wsb));
+        const uint8_t * wsb = Q4 ? W + 144 * s : W;
+        asm volatile("" : "+s"(wsb));
 #pragma unroll
-            for (int k = 0; k < 5; ++k) lds_dma16(wsb + wrow[k], L.w + 1024 * k);
+        for (int k = 0; k < NCW; ++k) {
+            if constexpr (Q4) lds_dma16(wsb + wrow[k], L.w + 1024 * k);
+            else lds_dma16(wsb + min((wrow[k] + 82u * (uint32_t)s) & ~15u, last), L.w + 1024 * k);
         }
     };
     copy_w(0);                                                  // before the pairs are known
@@ -599,23 +604,14 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
     // ---- this lane's rows: local row 32 wave + 16 rs + l16 is gate row
     // 64 rb + r (r < 64) or up row F + 64 rb + r - 64, clamped into the slab
     // (rows past n_ff are computed and discarded)
-    uint32_t voff[2], rowpar[2];
+    uint32_t voff[2];
 #pragma unroll
     for (int rs = 0; rs < 2; ++rs) {
         const int r = 32 * wave + 16 * rs + l16;
         const int gi = min(64 * rb + (r & 63), F - 1);
         const int row = r < 64 ? gi : F + gi;
         voff[rs] = (uint32_t)row * rbytes;
-        rowpar[rs] = (voff[rs] >> 1) & 1u;                      // row start mod 4, halved (slabs are 16-aligned)
     }
-    Iq2Raw wi[Q4 ? 1 : 2];
-    auto load_rows = [&](int s) {
-        if constexpr (!Q4) {
-#pragma unroll
-            for (int rs = 0; rs < 2; ++rs) iq2_raw_load(wi[rs], wr, voff[rs], rowpar[rs], s, q);
-        }
-    };
-
     f4 y[2][NT];
 #pragma unroll
     for (int rs = 0; rs < 2; ++rs)
@@ -659,7 +655,7 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
         float dr[2], mr[2];
         uint32_t sh03[2], sl03[2], sh47[2], sl47[2];         // Q4_K
         uint2 qs8[2], sg8[2];                                // IQ2_S
-        uint32_t qh2[2], sc2[2];
+        uint32_t qh2[2], sc2[2], d2[2];
         h8 bm[2];
         u32x4 hdr4[Q4 ? 2 : 1], nib[Q4 ? 2 : 1][2];
         if constexpr (Q4) {
@@ -674,6 +670,29 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
                 // in registers before the next super-block lands in their room
 #pragma unroll
                 for (int rs = 0; rs < 2; ++rs) asm volatile("" : "+v"(hdr4[rs]), "+v"(nib[rs][0]), "+v"(nib[rs][1]));
+                copy_w(s + 1);
+            }
+        } else {
+            // the lane's groups 4q .. 4q + 3: grid entries 8q .. 8q + 7.  The
+            // qs and sign dwords are 2-aligned: read as the aligned dwords
+            // around them and shifted into place
+#pragma unroll
+            for (int rs = 0; rs < 2; ++rs) {
+                const int at = (16 * rs + l16) * 96 + (int)((voff[rs] + 82u * (uint32_t)s) & 15u);
+                const uint32_t * v = reinterpret_cast<const uint32_t *>(L.w + ((at + 2) & ~3) + 8 * q);
+                const uint32_t sh = 8u * (uint32_t)((at + 2) & 2);
+                const uint32_t a0 = v[0], a1 = v[1], a2 = v[2], b0 = v[8], b1 = v[9], b2 = v[10];
+                d2[rs] = *reinterpret_cast<const uint16_t *>(L.w + at);
+                qh2[rs] = *reinterpret_cast<const uint16_t *>(L.w + at + 66 + 2 * q);     // 2 bits per entry
+                sc2[rs] = *reinterpret_cast<const uint16_t *>(L.w + at + 74 + 2 * q);     // 4 bits per group
+                qs8[rs] = make_uint2(__builtin_amdgcn_alignbit(a1, a0, sh), __builtin_amdgcn_alignbit(a2, a1, sh));
+                sg8[rs] = make_uint2(__builtin_amdgcn_alignbit(b1, b0, sh), __builtin_amdgcn_alignbit(b2, b1, sh));
+            }
+            if constexpr (MORE) {
+#pragma unroll
+                for (int rs = 0; rs < 2; ++rs)
+                    asm volatile("" : "+v"(d2[rs]), "+v"(qh2[rs]), "+v"(sc2[rs]), "+v"(qs8[rs].x), "+v"(qs8[rs].y),
+                                      "+v"(sg8[rs].x), "+v"(sg8[rs].y));
                 copy_w(s + 1);
             }
         }
@@ -702,23 +721,12 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
                     bm[rs][2 * i + 1] = mv.y;
                 }
             } else {
-                const Iq2Raw & w = wi[rs];
-                dr[rs] = h2f((w.d >> w.sh_d) & 0xFFFFu);
+                dr[rs] = h2f(d2[rs]);
                 mr[rs] = 0.0f;
-                // this lane's groups 4q .. 4q + 3: grid entries 8q .. 8q + 7
-                qs8[rs] = make_uint2(__builtin_amdgcn_alignbit(w.qs.y, w.qs.x, w.sh_q),
-                                     __builtin_amdgcn_alignbit(w.qs.z, w.qs.y, w.sh_q));
-                sg8[rs] = make_uint2(__builtin_amdgcn_alignbit(w.sg.y, w.sg.x, w.sh_q),
-                                     __builtin_amdgcn_alignbit(w.sg.z, w.sg.y, w.sh_q));
-                qh2[rs] = (w.qh >> w.sh_h) & 0xFFFFu;               // 2 bits per entry
-                sc2[rs] = (w.sc >> w.sh_h) & 0xFFFFu;               // 4 bits per group
 #pragma unroll
                 for (int j = 0; j < 8; ++j) bm[rs][j] = (_Float16)0.0f;
             }
         }
-
-        // ---- the next super-block's IQ2_S rows in flight during this one's MFMAs
-        if constexpr (MORE) load_rows(s + 1);
 
         // ---- slice by slice: expand, then every tile's MFMAs; a three-tile
         // group takes its row tiles one after the other (with the accumulators
@@ -823,7 +831,6 @@ __device__ __forceinline__ void pf_gu2_group(const PfParams & p, const PfTile & 
     };
 
     copy_in(0, L.x0, L.mb0, L.d80);
-    load_rows(0);
     int s = 0;
     for (; s + 2 < NSB; s += 2) {
         step(s, L.x0, L.mb0, L.d80, L.x1, L.mb1, L.d81, std::true_type{});
@@ -894,10 +901,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3, 3))) void
     __shared__ __align__(16) _Float16 mb1[G2_MBT * 16];
     __shared__ __align__(16) float d80[128];
     __shared__ __align__(16) float d81[128];
-    __shared__ __align__(16) uint8_t w[(WG / 64) * G2_WROW];
+    __shared__ __align__(16) uint8_t wa[G2_WA];
+    __shared__ __align__(16) uint8_t wb[G2_WB];
     __shared__ int tok[G2_TOK], pair[G2_TOK];
-    const Gu2Lds sm = {x0, x1, w + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * G2_WROW, mb0, mb1, d80, d81,
-                       reinterpret_cast<uint2 *>(w), reinterpret_cast<u32x4 *>(w + 1024 * 8), tok, pair};
+    Gu2Lds sm = {x0, x1, nullptr, mb0, mb1, d80, d81, reinterpret_cast<uint2 *>(wb),
+                 reinterpret_cast<u32x4 *>(wb + 1024 * 8), tok, pair};
     const int g = 8 * blockIdx.z + blockIdx.x, rb = blockIdx.y;
     const PfTile tile = load_tile(p.gtiles, p.max_gtiles, g);
     if (g >= *p.n_gtiles) return;
@@ -906,13 +914,16 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3, 3))) void
     const int nt = (tile.n + 15) >> 4;
     if (tile.n > G2_TOK) return;
     static_assert(G2_TOK == 48, "three tile counts");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (wt == T_Q4_K) {
+        sm.w = (wave < 2 ? wa : wb) + (wave & 1) * G2_WROW;
         switch (nt) {
         case 1: pf_gu2_group<T_Q4_K, GSRC, 1>(p, tile, sm, rb); break;
         case 2: pf_gu2_group<T_Q4_K, GSRC, 2>(p, tile, sm, rb); break;
         default: pf_gu2_group<T_Q4_K, GSRC, 3>(p, tile, sm, rb); break;
         }
     } else {
+        sm.w = wa + wave * G2_IQROW;
         switch (nt) {
         case 1: pf_gu2_group<T_IQ2_S, GSRC, 1>(p, tile, sm, rb); break;
         case 2: pf_gu2_group<T_IQ2_S, GSRC, 2>(p, tile, sm, rb); break;
