@@ -819,6 +819,20 @@ __device__ __forceinline__ void dn_pair_load(DnPair & q, const uint8_t * src) {
     }
 }
 
+// the same of either format, without a branch (lanes of one wave hold rows of
+// both): the last 12 bytes of the pair hold its last dwords
+__device__ __forceinline__ void dn_pair_load_any(DnPair & q, const uint8_t * src, bool q5) {
+    const u32x4a * s4 = reinterpret_cast<const u32x4a *>(src);
+    const u32x4a a = s4[0], b = s4[1];
+    const uint32_t * s1 = reinterpret_cast<const uint32_t *>(src + (q5 ? 32 : 24));
+    const uint32_t c0 = s1[0], c1 = s1[1], c2 = s1[2];
+    q.w[0] = a.x; q.w[1] = a.y; q.w[2] = a.z; q.w[3] = a.w;
+    q.w[4] = b.x; q.w[5] = b.y; q.w[6] = b.z; q.w[7] = b.w;
+    q.w[8] = q5 ? c0 : c2;
+    q.w[9] = c1;
+    q.w[10] = c2;
+}
+
 // the member activation's 32-block b from LDS: 32 int8 values, its scale
 // and its sum (q8_1: of the values, stored as fp16; q8_0: of the int8
 // values, exact)
@@ -992,21 +1006,16 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(1, 4))) void
     const int abytes = (int)p.yq_stride;                      // one quantised column, a multiple of 16
     const int NP = F / 64;                                    // block pairs per row
 
-    // 1. the columns' first loads, then the records
     const u32x4 * yq4 = reinterpret_cast<const u32x4 *>(p.yq);
     const int nch = P * (abytes / 16);
-    u32x4 col[DN_CL];
-#pragma unroll
-    for (int k = 0; k < DN_CL; ++k) col[k] = yq4[min((int)threadIdx.x + k * WG, nch - 1)];
-    {
-        const GroupInfo gi_in = p.ctl->groups[min((int)threadIdx.x, DEC_PMAX - 1)];
-        const int ngv = p.ctl->n_groups;
-        const float wv = p.w[min((int)threadIdx.x, P - 1)];
-        if (threadIdx.x == 0) s_ng = ngv;
-        if ((int)threadIdx.x < DEC_PMAX) s_wt[threadIdx.x] = (int)threadIdx.x < P ? wv : 0.0f;
-        for (int i = threadIdx.x; i < P * DEC_DN_MAXR; i += WG) (&s_y[0][0])[i] = 0.0f;
-        __syncthreads();
-        const int ng = max(0, min(s_ng, DEC_PMAX));
+    const int lrow = threadIdx.x / DN_LPR, lane16 = threadIdx.x % DN_LPR;
+    const int pl = min(lane16, NP - 1);
+    constexpr int DA = MT == 1 ? 2 : 8;                       // passes whose block pairs are in flight at once
+    constexpr int CL = MT == 1 ? 4 : DN_CL;
+    DnPair w[DA];
+    int kw[DA];
+    u32x4 col[CL];
+    auto table = [&](const GroupInfo & gi_in, int ng) {
         if ((int)threadIdx.x < ng) {
             const GroupInfo gi = validate_group(p, gi_in, ng, threadIdx.x);
             DnGroup d;
@@ -1024,46 +1033,85 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(1, 4))) void
                                  : 0;
             s_gi[threadIdx.x] = d;
         }
+    };
+    auto pair_load = [&](DnPair & q, int tier, const uint8_t * slab, uint32_t off) {
+        if constexpr (HD == CD) dn_pair_load<HD>(q, slab + off);
+        else if constexpr (MT == 1) dn_pair_load_any(q, slab + off, (tier == 0 ? HD : CD) == T_Q5_0);
+        else if (tier == 0) dn_pair_load<HD>(q, slab + off);
+        else dn_pair_load<CD>(q, slab + off);
+    };
+    if constexpr (MT == 1) {
+        // 1. every lane reads the records of its passes' groups and starts
+        // their block pairs at once, with no barrier between (a record past the
+        // call's groups sends the loads to any valid row and is not used); the
+        // table of the groups and the columns meet the other lanes at one
+        // barrier, while the rows are on their way
+        uint2 rec[DA];                                        // tier, idx
+#pragma unroll
+        for (int q = 0; q < DA; ++q)
+            rec[q] = *reinterpret_cast<const uint2 *>(p.ctl->groups + min((q * DN_RPP + lrow) >> lg2r, P - 1));
+        const GroupInfo gi_in = p.ctl->groups[min((int)threadIdx.x, DEC_PMAX - 1)];
+        const int ng = max(0, min(p.ctl->n_groups, DEC_PMAX));
+        const float wv = p.w[min((int)threadIdx.x, P - 1)];
+#pragma unroll
+        for (int k = 0; k < CL; ++k) col[k] = yq4[min((int)threadIdx.x + k * WG, nch - 1)];
+        __builtin_amdgcn_sched_barrier(0);                    // all of them issued before the first is waited for
+#pragma unroll
+        for (int q = 0; q < DA; ++q) {
+            const int tier = (int)rec[q].x, idx = (int)rec[q].y;
+            const bool hot = tier == 0 && idx >= 0 && idx < p.k_slots, cold = tier == 1 && idx >= 0 && idx < p.n_expert;
+            const uint8_t * slab = hot ? p.hot_dn + (uint64_t)idx * p.hot_dn_stride
+                                       : p.cold_dn + (uint64_t)(cold ? idx : 0) * p.cold_dn_stride;
+            const int bb = blk_bytes(hot ? HD : CD), r = min((q * DN_RPP + lrow) & (R - 1), max(nr - 1, 0));
+            kw[q] = hot ? 0 : 1;
+            pair_load(w[q], kw[q], slab, (uint32_t)(r0 + r) * (uint32_t)((F / 32) * bb) + (uint32_t)(pl * 2 * bb));
+        }
+        if (threadIdx.x == 0) s_ng = ng;
+        if ((int)threadIdx.x < DEC_PMAX) s_wt[threadIdx.x] = (int)threadIdx.x < P ? wv : 0.0f;
+        for (int i = threadIdx.x; i < P * DEC_DN_MAXR; i += WG) (&s_y[0][0])[i] = 0.0f;
+        table(gi_in, ng);
+    } else {
+        // 1. the columns' first loads, then the records
+#pragma unroll
+        for (int k = 0; k < CL; ++k) col[k] = yq4[min((int)threadIdx.x + k * WG, nch - 1)];
+        const GroupInfo gi_in = p.ctl->groups[min((int)threadIdx.x, DEC_PMAX - 1)];
+        const int ngv = p.ctl->n_groups;
+        const float wv = p.w[min((int)threadIdx.x, P - 1)];
+        if (threadIdx.x == 0) s_ng = max(0, min(ngv, DEC_PMAX));
+        if ((int)threadIdx.x < DEC_PMAX) s_wt[threadIdx.x] = (int)threadIdx.x < P ? wv : 0.0f;
+        for (int i = threadIdx.x; i < P * DEC_DN_MAXR; i += WG) (&s_y[0][0])[i] = 0.0f;
+        __syncthreads();
+        table(gi_in, s_ng);
+        __syncthreads();
     }
-    __syncthreads();
-    const int ng = max(0, min(s_ng, DEC_PMAX));
-    const int rows = ng << lg2r, passes = (rows + DN_RPP - 1) / DN_RPP;
-    const int lrow = threadIdx.x / DN_LPR, lane16 = threadIdx.x % DN_LPR;
-    const int pl = min(lane16, NP - 1);
-
     // the block pair of this lane in pass `ps` (a clamped, valid address when
     // the lane has none)
-    auto pair_src = [&](int ps, int * kind) {
+    auto load = [&](DnPair & q, int ps, int ng, int * kind) {
         const int k = ps * DN_RPP + lrow, s = min(k >> lg2r, max(ng - 1, 0)), r = min(k & (R - 1), max(nr - 1, 0));
         const DnGroup & d = s_gi[s];
         *kind = d.tier == 0 ? 0 : 1;
-        const uint8_t * base = d.tier == 0 ? p.hot_dn : p.cold_dn;
-        return base + d.row0 + (uint64_t)r * d.rb + (uint64_t)pl * (blk_bytes(d.tier == 0 ? HD : CD) * 2);
+        pair_load(q, *kind, (d.tier == 0 ? p.hot_dn : p.cold_dn) + d.row0,
+                  (uint32_t)r * (uint32_t)d.rb + (uint32_t)(pl * blk_bytes(d.tier == 0 ? HD : CD) * 2));
     };
-    auto load = [&](DnPair & q, int ps, int * kind) {
-        const uint8_t * src = pair_src(ps, kind);
-        if (*kind == 0) dn_pair_load<HD>(q, src);
-        else dn_pair_load<CD>(q, src);
-    };
-    // every pass's block pairs in flight at once (up to DA passes; later ones
-    // are loaded when they come)
-    constexpr int DA = MT == 1 ? 2 : 8;
-    DnPair w[DA];
-    int kw[DA];
+    // later passes than DA are loaded when they come
+    if constexpr (MT > 1) {
+        const int rows = s_ng << lg2r, passes = (rows + DN_RPP - 1) / DN_RPP;
 #pragma unroll
-    for (int q = 0; q < DA; ++q) {
-        kw[q] = 0;
-        if (q < passes) load(w[q], q, &kw[q]);
+        for (int q = 0; q < DA; ++q) {
+            kw[q] = 0;
+            if (q < passes) load(w[q], q, s_ng, &kw[q]);
+        }
     }
 
     // 2. the columns into LDS
 #pragma unroll
-    for (int k = 0; k < DN_CL; ++k) {
+    for (int k = 0; k < CL; ++k) {
         const int i = threadIdx.x + k * WG;
         if (i < nch) reinterpret_cast<u32x4 *>(smem)[i] = col[k];
     }
-    for (int i = threadIdx.x + DN_CL * WG; i < nch; i += WG) reinterpret_cast<u32x4 *>(smem)[i] = yq4[i];
+    for (int i = threadIdx.x + CL * WG; i < nch; i += WG) reinterpret_cast<u32x4 *>(smem)[i] = yq4[i];
     __syncthreads();
+    const int ng = s_ng, rows = ng << lg2r, passes = (rows + DN_RPP - 1) / DN_RPP;
 
     // 3. the passes: DN_RPP rows each, one row per DN_LPR lanes
     auto pass = [&](const DnPair & cur, int kc, int ps) {
@@ -1103,7 +1151,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(1, 4))) void
     for (int ps = DA; ps < passes; ++ps) {
         DnPair t;
         int kt = 0;
-        load(t, ps, &kt);
+        load(t, ps, ng, &kt);
         pass(t, kt, ps);
     }
     __syncthreads();
