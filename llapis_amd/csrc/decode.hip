@@ -512,10 +512,9 @@ __device__ __forceinline__ void item_dot(const uint8_t * sm, int wb, int n_mem, 
             }
         }
     }
+    static_assert(LPR == 16, "a row of 16 lanes");
 #pragma unroll
-    for (int c = 0; c < MT; ++c)
-#pragma unroll
-        for (int o = LPR / 2; o >= 1; o >>= 1) acc[c] += __shfl_xor(acc[c], o, LPR);
+    for (int c = 0; c < MT; ++c) acc[c] = row16_sum_f(acc[c]);
 }
 
 // Wave w stages and dots four rows of an item: rows 4 (w mod 8) .. + 3 of the
@@ -1135,10 +1134,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(1, 4))) void
                 }
             }
         }
+        static_assert(DN_LPR == 16, "a row of 16 lanes");
 #pragma unroll
-        for (int c = 0; c < MT; ++c)
-#pragma unroll
-            for (int o = DN_LPR / 2; o >= 1; o >>= 1) acc[c] += __shfl_xor(acc[c], o, DN_LPR);
+        for (int c = 0; c < MT; ++c) acc[c] = row16_sum_f(acc[c]);
         if (live && lane16 == 0) {
 #pragma unroll
             for (int c = 0; c < MT; ++c)

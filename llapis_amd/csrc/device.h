@@ -232,6 +232,16 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {
     const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
+// the same of a float, the sums of a butterfly over lane distances 8, 4, 2, 1
+// (rotations within the row: after the first the values repeat every 8 lanes,
+// and so on): no LDS round trips
+__device__ __forceinline__ float row16_sum_f(float v) {
+    v += dpp_f<0x128>(v, v);        // row_ror:8
+    v += dpp_f<0x124>(v, v);
+    v += dpp_f<0x122>(v, v);
+    v += dpp_f<0x121>(v, v);
+    return v;
+}
 // sum over each row of 16 lanes, in every lane of the row
 __device__ __forceinline__ int row16_sum(int v) {
     v += dpp_i<0xB1>(0, v);
