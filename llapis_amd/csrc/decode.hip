@@ -167,10 +167,16 @@ __device__ __forceinline__ int wave_max_i(int v) {
 
 constexpr int DEC_KMAX = 16;    // top_k of a decode call, at most
 
-// one wave's scratch for ordering its selected entries
+// one wave's scratch for gathering its selected entries
 struct SelScratch {
     int key[DEC_KMAX], idx[DEC_KMAX];
 };
+
+__device__ __forceinline__ double readlane_d(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
 
 // Softmax + top-K of one token in one wave, from its logits in registers
 // (v[j] = entry lane + 64 j; entries at or past E are ignored), as ggml's CPU
@@ -181,11 +187,12 @@ struct SelScratch {
 // The K-th largest probability is found by bisection over its bits (the
 // largest t with at least K probabilities >= t: one ballot count per step),
 // stopping early once exactly K entries are >= t; the entries above it and
-// the lowest-indexed ones equal to it are taken, and each taken entry's rank
-// (larger first, then the lower index) counts the taken entries before it,
-// read from the lanes.  No cross-lane shuffles in the loops; one LDS round
-// trip orders the K entries.  ids and weights go to LDS when `wr`; entries
-// past the valid ones (K > E) get id -1 and weight 0.
+// the lowest-indexed ones equal to it are taken, gathered in lanes 0 .. K - 1
+// and ranked there against each other (ranking them where they lie, in a loop
+// over their lanes, took 1450 cycles of the selection's 4600, the sum's loop
+// 780, now 300).  Taking the maximum K times instead takes 3040 cycles against
+// 2560 for the bisection and those ranks.  ids and weights go to LDS when
+// `wr`; entries past the valid ones (K > E) get id -1 and weight 0.
 template <int NJ>
 __device__ __forceinline__ void select_topk(const float (&v)[4], int E, int K, int * s_ids, float * s_w, bool wr,
                                             SelScratch & sc) {
@@ -249,36 +256,50 @@ __device__ __forceinline__ void select_topk(const float (&v)[4], int E, int K, i
             }
         }
     }
-    // ranks of this lane's taken entries
-    int rank[NJ];
+    // the taken entries in index order in lanes 0 .. kk - 1, by LDS
+    int before = 0;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) rank[j] = 0;
-#pragma unroll
-    for (int jj = 0; jj < NJ; ++jj) {
-        uint64_t m = sel[jj];
-        while (m) {
-            const int l = (int)__builtin_ctzll(m);
-            m &= m - 1;
-            const int kq = __builtin_amdgcn_readlane(q[jj], l), ki = l + 64 * jj;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-                rank[j] += (kq > q[j] || (kq == q[j] && ki < lane + 64 * j)) ? 1 : 0;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int j = 0; j < NJ; ++j) {
         if ((sel[j] >> lane) & 1) {
-            sc.key[rank[j]] = q[j];
-            sc.idx[rank[j]] = lane + 64 * j;
+            const int at = before + __popcll(sel[j] & lanes_below());
+            if (at < DEC_KMAX) {
+                sc.key[at] = q[j];
+                sc.idx[at] = lane + 64 * j;
+            }
         }
+        before += __popcll(sel[j]);
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int mine = min(lane, DEC_KMAX - 1);
-    const int myid = lane < kk ? sc.idx[mine] : -1;
-    const int mykey = lane < kk ? sc.key[mine] : 0;
+    int myid = lane < kk ? sc.idx[mine] : -1;
+    int mykey = lane < kk ? sc.key[mine] : 0;
+    // each one's rank: the entries larger than it, and the equal ones before
+    // it; then entry k to lane k (a lane past them keeps its own)
+    int rank = 0;
+    auto count = [&](int k) {
+        const int o = __builtin_amdgcn_readlane(mykey, k);
+        rank += k < kk && (o > mykey || (o == mykey && k < lane)) ? 1 : 0;
+    };
+#pragma unroll
+    for (int k = 0; k < DEC_KMAX / 2; ++k) count(k);
+    if (K > DEC_KMAX / 2) {
+#pragma unroll
+        for (int k = DEC_KMAX / 2; k < DEC_KMAX; ++k) count(k);
+    }
+    if (lane >= kk) rank = lane;
+    myid = __builtin_amdgcn_ds_permute(4 * rank, myid);
+    mykey = __builtin_amdgcn_ds_permute(4 * rank, mykey);
+    // the sum in order; entries past the taken ones add zeros
+    const double kd = (double)__int_as_float(mykey);
     double sum = 0.0;
-    for (int k = 0; k < kk; ++k) sum += (double)__int_as_float(__builtin_amdgcn_readlane(mykey, k));
+#pragma unroll
+    for (int k = 0; k < DEC_KMAX / 2; ++k) sum += readlane_d(kd, k);
+    if (K > DEC_KMAX / 2) {
+#pragma unroll
+        for (int k = DEC_KMAX / 2; k < DEC_KMAX; ++k) sum += readlane_d(kd, k);
+    }
     float sf = (float)sum;
     if (sf < 6.103515625e-5f) sf = 6.103515625e-5f;
     if (wr && lane < K) {
@@ -526,30 +547,30 @@ __device__ __forceinline__ void item_dot(const uint8_t * sm, int wb, int n_mem, 
 // of the next step as soon as its dots are done.
 template <int MT>
 __device__ __forceinline__ int gu_wave_half(int h) {
-    return gu_halves<MT>() == 2 ? (int)(threadIdx.x >> 9) : h;
+    return gu_halves<MT>() == 2 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 9)) : h;
 }
 template <int HT, int CT, int MT>
 __device__ __forceinline__ Span gu_wave_span(const DecParams & p, const GroupInfo & gi, int j, int h) {
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     return make_span(gi, gu_wave_half<MT>(h) * p.n_ff + DEC_GU_BLK * j + 4 * (wave & 7), 4, p.d_model, HT, CT,
                      p.hot_gu, p.hot_gu_stride, p.cold_gu, p.cold_gu_stride, p.logits);
 }
 template <int HT, int CT, int MT>
 __device__ __forceinline__ void gu_wave_load(const DecParams & p, const GroupInfo & gi, int j, int h, uint8_t * smem) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const Span sp = gu_wave_span<HT, CT, MT>(p, gi, j, h);
     uint8_t * dst = smem + wave * (p.w_lds_gu / 8);
-    for (int k = 0; 64 * k < sp.nch; ++k) {                // wave-uniform bound
-        const int c = 64 * k + lane;
-        if (c < sp.nch) lds_dma16(sp.src + c, dst + 1024 * k);
-    }
+    const uint8_t * src = reinterpret_cast<const uint8_t *>(sp.src);
+    int k = 0;
+    for (; 64 * (k + 1) <= sp.nch; ++k) lds_dma16(src + (uint32_t)(1024 * k + 16 * lane), dst + 1024 * k);   // wave-uniform bound
+    if (64 * k + lane < sp.nch) lds_dma16(src + (uint32_t)(1024 * k + 16 * lane), dst + 1024 * k);
 }
 // the four rows' dots against the members' columns: acc[c], complete in
 // every lane of the row
 template <int WT, int HT, int CT, int AM, int MT>
 __device__ __forceinline__ void gu_wave_dots(const DecParams & p, const GroupInfo & gi, int j, int h,
                                              const uint8_t * smem, const ActView * av, int grid_off, float * acc) {
-    const int wave = threadIdx.x >> 6, r = (threadIdx.x >> 4) & 3;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), r = (threadIdx.x >> 4) & 3;
     const bool live = gi.tier < 2 && gi.n_mem > 0;
     const Span sp = gu_wave_span<HT, CT, MT>(p, gi, j, h);
     const int wb = wave * (p.w_lds_gu / 8) + sp.off + r * sp.rb;
@@ -623,8 +644,13 @@ void k_dec_gate_up(const DecParams p) {
     __shared__ GroupInfo s_grp[DEC_PMAX];     // kept for every item of the workgroup
     __shared__ int s_ng;
     __shared__ float s_y[2][2 * GU_HR][MT];   // by item parity (the epilogue has one barrier)
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int T = p.T, K = p.top_k, E = p.n_expert, d_in = p.d_model, F = p.n_ff;
+    // item / NBLK as (item per_blk) >> 16: exact below 64 groups x 32 blocks
+    // (item (per_blk NBLK - 65536) < 65536); formed here, while nothing waits for it
+    const int NBLK = F / DEC_GU_BLK;
+    uint32_t per_blk = (65536u + (uint32_t)NBLK - 1u) / (uint32_t)NBLK;
+    asm volatile("" : "+s"(per_blk));
 
     // 1. the routing's loads, none under a lane condition: the logits of this
     //    wave's token (waves below T), the residency mirrors
@@ -697,20 +723,31 @@ void k_dec_gate_up(const DecParams p) {
     __syncthreads();
     if (wave == 0) build_groups(p, s_ids, s_grp, &s_ng, s_res[0], s_res[1], s_res[2], s_first, s_tm, s_first);
     __syncthreads();
-    const int ng = max(0, min(s_ng, DEC_PMAX));
-    const int NBLK = F / DEC_GU_BLK, n_items = ng * NBLK;
+    const int ng = max(0, min(__builtin_amdgcn_readfirstlane(s_ng), DEC_PMAX));
+    const int n_items = ng * NBLK;
     if ((int)blockIdx.x >= n_items) return;   // workgroup-uniform (workgroup 0 always has item 0)
     // workgroup b takes the items at positions b, b + grid, ...; with more
     // items than workgroups, positions past the grid (second items) take the
     // cheapest items and the first workgroups (the ones with a second item)
     // the next cheapest (the groups taken in .ord order, cheapest first)
     const int G = (int)gridDim.x, shift = max(0, n_items - G);
+    // An item's group is the same in every lane: its fields go to scalar
+    // registers, and with them the addresses and bounds of its rows (in vector
+    // registers they, and a division, cost 2500 cycles between the routing and
+    // the first weight's load)
     auto item = [&](int pos, int * jo) {
         const int it = pos >= G ? pos - G : pos + shift;
-        const int k = it / NBLK;
-        const int g = max(0, min(s_grp[k].ord, ng - 1));
+        const int k = (int)(((uint32_t)it * per_blk) >> 16);
+        const int g = MT == 1 ? k : max(0, min(__builtin_amdgcn_readfirstlane(s_grp[k].ord), ng - 1));
         *jo = it - k * NBLK;
-        return validate_group(p, s_grp[g], ng, g);
+        GroupInfo gi;
+        gi.tier = __builtin_amdgcn_readfirstlane(s_grp[g].tier);
+        gi.idx = __builtin_amdgcn_readfirstlane(s_grp[g].idx);
+        gi.n_mem = __builtin_amdgcn_readfirstlane(s_grp[g].n_mem);
+        gi.ord = 0;
+#pragma unroll
+        for (int c = 0; c < DEC_MAXT; ++c) gi.mem[c] = c < MT ? __builtin_amdgcn_readfirstlane(s_grp[g].mem[c]) : 0;
+        return validate_group(p, gi, ng, g);
     };
 
     // 3. the first item's weights (the routing's scratch is dead: the barrier above)
@@ -737,7 +774,10 @@ void k_dec_gate_up(const DecParams p) {
     while (true) {
         ActView av[MT];
 #pragma unroll
-        for (int c = 0; c < MT; ++c) act_layout(d_in, a0 + max(0, min(member(gi, c) / K, T - 1)) * abytes, &av[c]);
+        for (int c = 0; c < MT; ++c) {
+            const int m = member(gi, c), t = (m >= K) + (m >= 2 * K) + (m >= 3 * K);       // m / K, m < 4 K
+            act_layout(d_in, a0 + min(t, T - 1) * abytes, &av[c]);
+        }
         __builtin_amdgcn_s_waitcnt(0);                    // this wave's rows have landed
         float acc[MT];
         if (gi.tier == 0) gu_wave_dots<HT, HT, CT, AM, MT>(p, gi, j, h, smem, av, grid_off, acc);
