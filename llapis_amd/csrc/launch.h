@@ -167,7 +167,7 @@ struct PfParams {
                                          //   q8_1: per-32 d sum(q) as hi, lo
     int act_mode;                        // AM_CPU (q8_K / q8_0) or AM_Q8_1
     _Float16 * xh;                       // [T][d_model / 256][512] q8_1 values d q as fp16 hi (256), lo (256)
-    _Float16 * ah;                       // [P][n_ff] down activations d8 q: fp16 high part
+    _Float16 * ah;                       // [P][n_ff] down activations d8 q (each 32-block in dn_pos order): fp16 high part
     _Float16 * al;                       // [P][n_ff]                        exact remainder
     float * ydn;                         // [P][d_model]
     int32_t * rc_counts;                 // [n_expert] routed pairs per expert, or NULL

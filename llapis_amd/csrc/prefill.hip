@@ -17,18 +17,18 @@
 //                  (pf_quant_x1: q8_1, as exact fp16 parts).
 //   k_pf_gate_up   grouped GEMM per (group, 64 gate rows + the 64 matching up
 //                  rows), on groups of its own (<= 48 pairs), the full groups
-//                  first, every row block of a group on one XCD.  Each super-block of weights
-//                  is expanded once into int8 MFMA operands and used for
-//                  every token of the group.  The sub-block scales are folded
+//                  first, every row block of a group on one XCD.  Each
+//                  super-block of weights is expanded once into int8 MFMA
+//                  operands and used for every token of the group.  The sub-block scales are folded
 //                  into the weights: Q4_K's 6-bit scale splits as 8 sh + sl,
 //                  so q sh and q sl (<= 105) are int8 and two accumulators
 //                  give sum_j sc_j dot_j exactly; IQ2_S's grid * (2 ls + 1)
 //                  (<= 1333) splits as 64 h + l.  The Q4_K mins term is one
 //                  exact fp16 MFMA against the split per-32 sums.  Scales
 //                  d_w * d8 are applied once per super-block in fp32.  The
-//                  load unit copies the next super-block's activations (and
-//                  Q4_K rows) into LDS while the current one is used; IQ2_S
-//                  rows go straight to registers.  The epilogue pairs gate
+//                  load unit copies the next super-block's activations and
+//                  rows into LDS while the current one is used.  The
+//                  epilogue pairs gate
 //                  row i with up row n_ff + i: GEGLU and the q8_0
 //                  quantisation of the down activations happen here, so the
 //                  gate_up outputs never go to memory; each down activation
@@ -45,8 +45,9 @@
 //                  need a per-block fp32 rescale by d_w d8 (three VALU
 //                  operations per output and block), which made that variant
 //                  VALU-bound at several times this one's time.  K runs in
-//                  chunks of two blocks, copied into LDS by the load unit one
-//                  chunk ahead; every row block of a group on one XCD.
+//                  chunks of two blocks, activations and weight rows copied
+//                  into LDS by the load unit one step ahead; every row block
+//                  of a group on one XCD.
 // The combine is the generic k_combine.
 #include <hip/hip_ext.h>
 
@@ -1640,17 +1641,16 @@ void launch_gu(int gelu, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const PfPa
         else launch_pf(k_pf_gate_up<HT, CT, SRC_GEGLU_TABLE>, g2, s, e0, e1, p);
     }
 }
-// pairs per gate_up group of an expert in format t
-int gate_up_cap(int) { return G2_TOK; }
-// in the q8_1 mode (1 KB of activation parts per token and super-block)
+// pairs per q8_1 gate_up group of an expert in format t (1 KB of activation
+// parts per token and super-block)
 int gate_up_cap_q1(int t) { return t == T_Q4_K ? PF_TOK1Q4 : PF_TOK1IQ2; }
 }  // namespace
 
 hipError_t launch_prefill(const PfParams & p0, int hgu, int cgu, int hdn, int cdn, int gelu, hipStream_t s,
                           hipEvent_t * ev) {
     PfParams p = p0;
-    p.gcap[0] = p.act_mode == AM_Q8_1 ? gate_up_cap_q1(hgu) : gate_up_cap(hgu);
-    p.gcap[1] = p.act_mode == AM_Q8_1 ? gate_up_cap_q1(cgu) : gate_up_cap(cgu);
+    p.gcap[0] = p.act_mode == AM_Q8_1 ? gate_up_cap_q1(hgu) : G2_TOK;
+    p.gcap[1] = p.act_mode == AM_Q8_1 ? gate_up_cap_q1(cgu) : G2_TOK;
     hipEvent_t e[4] = {};
     if (ev)
         for (int i = 0; i < 4; ++i) e[i] = ev[i];
