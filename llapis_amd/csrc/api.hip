@@ -707,10 +707,10 @@ PfWs pf_layout(const llapis_moe_layer * L, int Tc) {
 
 PfWs pf_ws(const llapis_moe_layer * L, int32_t T, uint64_t ws_bytes = ~uint64_t(0)) {
     const int K = std::max(1, L->top_k);
-    const int most = std::max(1, PF_MAX_PAIRS / K), least = std::min<int>(T, PF_MIN_PAIRS / K);
-    const int chunks = (T + most - 1) / most;
-    const PfWs w = pf_layout(L, chunks == 1 ? T : std::min(most, ((T + chunks - 1) / chunks + 63) / 64 * 64));
-    return w.total <= ws_bytes ? w : pf_layout(L, least);
+    const int64_t most = std::max(1, PF_MAX_PAIRS / K), least = std::min<int64_t>(T, PF_MIN_PAIRS / K);
+    const int64_t chunks = (T + most - 1) / most;
+    const PfWs w = pf_layout(L, (int)(chunks == 1 ? T : std::min(most, ((T + chunks - 1) / chunks + 63) / 64 * 64)));
+    return w.total <= ws_bytes ? w : pf_layout(L, (int)least);
 }
 
 // the smallest workspace that llapis_moe_ffn accepts for T tokens on any path

@@ -170,13 +170,18 @@ def test_make_layer_pools_match_quantised_experts():
     assert lay.residency.is_hot(1) and not lay.residency.is_hot(0)
 
 
+def _desc(sp, k_slots):
+    desc = la._lib.LlapisMoeLayer()
+    desc.d_model, desc.n_ff, desc.n_expert, desc.top_k, desc.k_slots = sp.d_model, sp.n_ff, sp.n_expert, sp.top_k, k_slots
+    desc.hot_gu_type, desc.hot_dn_type, desc.cold_gu_type, desc.cold_dn_type = Q4_K, Q5_0, IQ2_S, IQ4_NL
+    return desc
+
+
 def test_workspace_sizes():
     import ctypes as C
     lib = la.lib()
     sp = LayerSpec()
-    desc = la._lib.LlapisMoeLayer()
-    desc.d_model, desc.n_ff, desc.n_expert, desc.top_k, desc.k_slots = sp.d_model, sp.n_ff, sp.n_expert, sp.top_k, 57
-    desc.hot_gu_type, desc.hot_dn_type, desc.cold_gu_type, desc.cold_dn_type = Q4_K, Q5_0, IQ2_S, IQ4_NL
+    desc = _desc(sp, 57)
     sizes = [int(lib.llapis_moe_ffn_workspace_size(C.byref(desc), T)) for T in (1, 2, 4, 5, 64, 512)]
     assert all(b > a for a, b in zip(sizes, sizes[1:]))
     # at least the per-pair gate_up and down outputs in fp32
@@ -184,3 +189,14 @@ def test_workspace_sizes():
         assert b >= T * sp.top_k * (2 * sp.n_ff + sp.d_model) * 4
         assert b % 256 == 0
     assert int(lib.llapis_moe_ffn_workspace_size(C.byref(desc), 0)) == 0
+
+
+def test_workspace_size_of_the_longest_call():
+    """The largest token count there is: the generic path's outputs of every
+    pair decide (4 d_model + 8 n_ff bytes a pair; logits and ids are below 2 %
+    of that), and no 32-bit sum of the chunk layout wraps."""
+    import ctypes as C
+    desc = _desc(LayerSpec(), 57)
+    T = 2 ** 31 - 1
+    want = T * desc.top_k * (2 * desc.n_ff + desc.d_model) * 4
+    assert want <= int(la.lib().llapis_moe_ffn_workspace_size(C.byref(desc), T)) <= want * 1.02
