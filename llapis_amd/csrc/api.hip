@@ -670,11 +670,11 @@ bool decode_eligible(const llapis_moe_layer * L, int32_t T) {
 
 // prefill path (T > DEC_MAXT, either activation mode): tokens are processed in
 // chunks of Tc tokens; one chunk's scratch.  A chunk reads every routed
-// expert's weights, so a call is cut into as few chunks as PF_MAX_PAIRS
-// allows, of equal size (whole 64-token router tiles): 1900 tokens at top-8,
-// d_model 2816, every expert hot, take 1036 us as four 512-token chunks and
-// 566 us in one.  A workspace too small for that (one sized for a shorter
-// call) is served in chunks of PF_MIN_PAIRS / top_k tokens.
+// expert's weights, so a call is cut into as few chunks as PF_MAX_PAIRS and
+// the workspace allow, of equal size (whole 64-token router tiles): 1900
+// tokens at top-8, d_model 2816, every expert hot, take 1036 us as four
+// 512-token chunks and 566 us in one.  Chunks of PF_MIN_PAIRS / top_k tokens
+// (the whole call, if it is shorter) are the shortest.
 struct PfWs {
     uint64_t probs, ids, w, ntiles, sorted, tiles, gtiles, xq, xd, xm, xh, ah, al, ydn, parts, total;
     int Tc, max_tiles, max_gtiles;
@@ -705,18 +705,31 @@ PfWs pf_layout(const llapis_moe_layer * L, int Tc) {
     return w;
 }
 
-PfWs pf_ws(const llapis_moe_layer * L, int32_t T, uint64_t ws_bytes = ~uint64_t(0)) {
-    const int K = std::max(1, L->top_k);
-    const int64_t most = std::max(1, PF_MAX_PAIRS / K), least = std::min<int64_t>(T, PF_MIN_PAIRS / K);
-    const int64_t chunks = (T + most - 1) / most;
-    const PfWs w = pf_layout(L, (int)(chunks == 1 ? T : std::min(most, ((T + chunks - 1) / chunks + 63) / 64 * 64)));
-    return w.total <= ws_bytes ? w : pf_layout(L, (int)least);
+// tokens of the longest and of the shortest chunk a call of T tokens is cut into
+int pf_most(const llapis_moe_layer * L, int32_t T) {
+    return std::min<int32_t>(T, std::max(1, PF_MAX_PAIRS / std::max(1, L->top_k)));
+}
+int pf_least(const llapis_moe_layer * L, int32_t T) {
+    return std::min<int32_t>(T, PF_MIN_PAIRS / std::max(1, L->top_k));
+}
+
+// the layout of the fewest chunks that fit ws_bytes; if none do, the shortest chunks'
+PfWs pf_ws(const llapis_moe_layer * L, int32_t T, uint64_t ws_bytes) {
+    const int64_t most = pf_most(L, T), least = pf_least(L, T);
+    for (int64_t chunks = (T + most - 1) / most;; ++chunks) {
+        const int64_t Tc = chunks == 1 ? T : std::min(most, ((T + chunks - 1) / chunks + 63) / 64 * 64);
+        if (Tc <= least) break;
+        const PfWs w = pf_layout(L, (int)Tc);
+        if (w.total <= ws_bytes) return w;
+        if (Tc <= 64) break;
+    }
+    return pf_layout(L, (int)least);
 }
 
 // the smallest workspace that llapis_moe_ffn accepts for T tokens on any path
 uint64_t least_workspace(const llapis_moe_layer * L, int32_t T) {
     const uint64_t b = ffn_ws(L, T).total;
-    return std::max(b, T <= DEC_MAXT ? dec_ws(L, T).total : pf_ws(L, T, 0).total);
+    return std::max(b, T <= DEC_MAXT ? dec_ws(L, T).total : pf_layout(L, pf_least(L, T)).total);
 }
 
 bool prefill_eligible(const llapis_moe_layer * L, int32_t T) {
@@ -737,8 +750,10 @@ void llapis_set_tuning(int32_t key, int32_t value) {
 
 uint64_t llapis_moe_ffn_workspace_size(const llapis_moe_layer * L, int32_t n_tokens) {
     if (!L || n_tokens <= 0) return 0;
+    // a chunk layout grows with its tokens: this one holds the chunks of the
+    // call and of every shorter call
     uint64_t b = least_workspace(L, n_tokens);
-    if (n_tokens > DEC_MAXT) b = std::max(b, pf_ws(L, n_tokens).total);
+    if (n_tokens > DEC_MAXT) b = std::max(b, pf_layout(L, pf_most(L, n_tokens)).total);
     return b;
 }
 

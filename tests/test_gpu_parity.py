@@ -613,6 +613,48 @@ def test_prefill_in_a_workspace_of_a_shorter_call(gpu):
         assert torch.equal(a, b)
 
 
+def _chunks(dl, x, ws=None):
+    """(out, ids, w) of one call and the chunks it ran in (a profiled call
+    records one entry per chunk), in its own or the given workspace."""
+    torch = torch_mod()
+    lib, d, T, sp = la.lib(), dl.desc(), x.shape[0], dl.layer.spec
+    ws = dl.workspace(T) if ws is None else ws
+    out = torch.full((T, sp.d_model), float("nan"), device=x.device)
+    ids = torch.full((T, sp.top_k), -1, dtype=torch.int32, device=x.device)
+    w = torch.full((T, sp.top_k), float("nan"), device=x.device)
+    ms = (C.c_float * 5)()
+    lib.llapis_profile_enable(1)
+    try:
+        rc = lib.llapis_moe_ffn(C.byref(d), x.data_ptr(), None, T, out.data_ptr(), ids.data_ptr(), w.data_ptr(),
+                                ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        n = lib.llapis_profile_read(ms, 5)
+    finally:
+        lib.llapis_profile_enable(0)
+    assert rc == 0, lib.llapis_last_error()
+    return (out, ids, w), n
+
+
+def test_prefill_takes_the_fewest_chunks_that_fit(gpu):
+    """A 3000-token call (top_k 4: at most 4096 and at least 1024 tokens a
+    chunk) in workspaces sized for fewer tokens: one chunk, two of 1536
+    (1600 tokens' room), three (1024 tokens' room); the same bits each way.  A
+    workspace sized for more tokens than one chunk holds takes it in one."""
+    torch = torch_mod()
+    spec, T = SMALL, 3000
+    say(f"prefill T={T} chunks by workspace")
+    dl = la.DeviceLayer(_layer_case(spec, 91, 6, True), gpu)
+    x = torch.from_numpy(tokens(603, T, spec.d_model)).to(gpu)
+    want, n = _chunks(dl, x)
+    assert n == 1
+    for room, chunks in ((4200, 1), (1600, 2), (1024, 3)):
+        size = int(la.lib().llapis_moe_ffn_workspace_size(C.byref(dl.desc()), room))
+        got, n = _chunks(dl, x, torch.empty(size, dtype=torch.uint8, device=gpu))
+        say(f"  room for {room} tokens: {n} chunks")
+        assert n == chunks
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("n_ff", [32, 64, 96, 224, 320])
 @pytest.mark.parametrize("T", [5, 150])
 @pytest.mark.parametrize("act_mode,gelu_mode", [(la.ACT_CPU, la.GELU_TABLE), (la.ACT_Q8_1, la.GELU_TANH)])

@@ -200,3 +200,17 @@ def test_workspace_size_of_the_longest_call():
     T = 2 ** 31 - 1
     want = T * desc.top_k * (2 * desc.n_ff + desc.d_model) * 4
     assert want <= int(la.lib().llapis_moe_ffn_workspace_size(C.byref(desc), T)) <= want * 1.02
+
+
+@pytest.mark.parametrize("d_model,n_ff,n_expert,top_k", [(2816, 704, 128, 8), (2816, 64, 128, 2), (8192, 32, 256, 1),
+                                                         (256, 1024, 8, 8), (3072, 256, 256, 2), (512, 96, 300, 300)])
+def test_workspace_serves_every_shorter_call(d_model, n_ff, n_expert, top_k):
+    """A workspace sized for max_tokens is at least what any shorter call's
+    size asks for: around the decode limit, the shortest chunks (4096 pairs),
+    and one and two whole chunks of 16384 pairs."""
+    import ctypes as C
+    desc = _desc(LayerSpec(d_model=d_model, n_ff=n_ff, n_expert=n_expert, top_k=top_k), min(57, n_expert))
+    marks = [1, 4, 64, 4096 // top_k, 16384 // top_k, 2 * 16384 // top_k]
+    Ts = sorted({t for m in marks for t in (*range(m - 2, m + 3), m + 64, m + 300) if t > 0})
+    sizes = [int(la.lib().llapis_moe_ffn_workspace_size(C.byref(desc), t)) for t in Ts]
+    assert all(b >= a for a, b in zip(sizes, sizes[1:])), list(zip(Ts, sizes))
