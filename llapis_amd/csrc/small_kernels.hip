@@ -489,9 +489,13 @@ int router_parts_floats(int T, int E) { return RSPLIT * T * E; }
 hipError_t launch_router_mfma(const float * x, int T, const float * w_r, int d, int E, float * parts, hipStream_t s) {
     if (d % (16 * RSPLIT) != 0 || T <= 0 || E <= 0) return hipErrorInvalidValue;
     dim3 grid((T + RT - 1) / RT, (E + RT - 1) / RT, RSPLIT);
-    // the staged kernel's 100 KB leave room for one workgroup a CU: ahead where
-    // every workgroup finds one (256: 9.0 against 9.5 us), behind where they
-    // queue (960, 1900 tokens: 30 against 21 us)
+    // the staged kernel's 100 KB leave room for one workgroup a CU: behind
+    // wherever they queue (at d 2816, launches back to back: 288 workgroups
+    // 13.8 against 10.3 us, 384 14.0 / 10.7, 512 13.7 / 10.8, 768 19.2 / 14.8,
+    // 1024 24.5 / 18.4; the same at d 1024 .. 3072, by 1.25 to 1.6), and ahead
+    // on a few tokens (32 workgroups 5.8 / 6.0 us, 128 7.2 / 7.3) or where x
+    // and w_r come from memory (256 inside a layer 9.0 / 9.5; back to back, in
+    // the caches, 8.2 / 7.9)
     if (d / RSPLIT <= RKC_MAX && grid.x * grid.y * grid.z <= 256)
         hipLaunchKernelGGL(k_router_mfma_st, grid, dim3(WG), 0, s, x, T, w_r, d, E, d / RSPLIT, parts);
     else hipLaunchKernelGGL(k_router_mfma, grid, dim3(WG), 0, s, x, T, w_r, d, E, d / RSPLIT, parts);
