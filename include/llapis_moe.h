@@ -161,7 +161,19 @@ typedef struct llapis_moe_layer {
     int32_t * route_hits;
 } llapis_moe_layer;
 
-/* Device scratch the layer needs for n_tokens (bytes). */
+/* Device scratch (bytes) for calls of up to n_tokens tokens: enough for each
+ * of them to run in the fewest chunks.  More than 4 tokens run in chunks of at
+ * most 16384 routed pairs, each of which reads the weights of every expert it
+ * is routed to; a smaller workspace that holds a chunk of 4096 / top_k tokens
+ * (what is returned for that many) is accepted too, and the call takes the
+ * fewest chunks that fit.  (Only layers of more than 256 experts or slots, or
+ * n_ff above 4096, need the size of the whole call.)  A chunk takes
+ * about 5.1 d_model + 68 n_expert bytes a token and 4 d_model + 4 n_ff a
+ * routed pair.  At top-8 that is what the whole call's outputs would take in
+ * fp32 (4 d_model + 8 n_ff a pair: 258 MB for 1900 tokens at d_model 2816,
+ * n_ff 704, 128 experts); with few picks a token and a small n_ff it is up to
+ * twice as much (490 MB for 8192 tokens at d_model 3072, n_ff 256, 256
+ * experts, top-2, where 4096-pair chunks run in 243). */
 uint64_t llapis_moe_ffn_workspace_size(const llapis_moe_layer * L, int32_t n_tokens);
 
 /* out [T][d_model] = the layer applied to x [T][d_model] (the experts'
@@ -184,10 +196,14 @@ int32_t llapis_moe_ffn(const llapis_moe_layer * L, const float * x, const float 
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * call's scratch is a fixed device array of LLAPIS_NOALLOC_SCRATCH_BYTES in
  * the library, one per GPU, held until the process ends; nothing is
- * allocated.  A call whose llapis_moe_ffn_workspace_size exceeds it is
- * refused (-1, llapis_last_error() says how much it needs): at the
- * benchmark's shapes (d_model 2816, n_ff 704, 128 experts, top-8) that
- * admits batches of up to 61 tokens.  Nothing is launched to prepare the
+ * allocated.  The array has to hold the routed pairs' gate_up and down outputs
+ * in fp32 (8 n_ff + 4 d_model bytes a pair of the whole call, with the logits
+ * and the routing) and one chunk of 4096 / top_k tokens (the whole call, if
+ * it is shorter), not all that llapis_moe_ffn_workspace_size returns, which
+ * is for the fewest chunks.  A call that needs more is refused (-1,
+ * llapis_last_error() says how much it needs): at the benchmark's shapes
+ * (d_model 2816, n_ff 704, 128 experts, top-8) that admits batches of up to
+ * 61 tokens.  Nothing is launched to prepare the
  * array: every call writes each scratch word before it reads it, so the first
  * call may itself be captured in a HIP graph.  Every call on one GPU shares
  * that GPU's array and leaves its contents behind: calls that overlap on one
