@@ -85,6 +85,18 @@ def dual_k57(full, seed, router_seed=None):
     return lay
 
 
+def in_workspace_for(dl, n_tokens):
+    """dl with its calls in a workspace sized for n_tokens tokens: longer
+    prefill calls run in several chunks."""
+    import ctypes as C
+
+    import torch
+    size = int(la.lib().llapis_moe_ffn_workspace_size(C.byref(dl.desc()), n_tokens))
+    ws = torch.zeros(size, dtype=torch.uint8, device=dl.device)
+    dl.workspace = lambda T: ws
+    return dl
+
+
 def per_token_rel_l2(got, want):
     return np.array([rel_l2(got[t], want[t]) for t in range(got.shape[0])])
 

@@ -22,7 +22,7 @@ from pathlib import Path
 
 import llapis_amd as la
 from llapis_amd import _lib as L
-from helpers import FULL16, SMALL, check_layer_bars, layer, oracle_mode, rel_l2, tokens
+from helpers import FULL16, SMALL, check_layer_bars, in_workspace_for, layer, oracle_mode, rel_l2, tokens
 
 GOLD = Path(__file__).resolve().parent / "golden"
 
@@ -565,10 +565,10 @@ def check_flip_tolerant(got, want):
 
 
 def test_prefill_chunks_and_generic_agree(gpu, oracle):
-    """A batch longer than one prefill launch (split into chunks of
-    4096 / top_k tokens) against the generic path and the oracle."""
+    """A batch longer than its workspace's chunk (1100 tokens in the room of
+    1024: two chunks) against the generic path and the oracle."""
     torch = torch_mod()
-    spec = SMALL                                 # top_k 4: chunks of 1024 tokens
+    spec = SMALL                                 # top_k 4: chunks of 1024 tokens at the least
     T = 1100
     say(f"prefill chunks T={T}")
     lay = _layer_case(spec, 91, 6, True)
@@ -576,7 +576,7 @@ def test_prefill_chunks_and_generic_agree(gpu, oracle):
     x = tokens(600, T, spec.d_model)
     xd = torch.from_numpy(x).to(gpu)
     lib = la.lib()
-    out_p, ids_p, w_p = (t.clone() for t in dl.forward(xd))
+    out_p, ids_p, w_p = (t.clone() for t in in_workspace_for(la.DeviceLayer(lay, gpu), 1024).forward(xd))
     try:
         lib.llapis_set_tuning(2, 0)
         out_g, ids_g, w_g = (t.clone() for t in dl.forward(xd))
@@ -653,6 +653,50 @@ def test_prefill_takes_the_fewest_chunks_that_fit(gpu):
         say(f"  room for {room} tokens: {n} chunks")
         assert n == chunks
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("act_mode,gelu_mode", [(la.ACT_CPU, la.GELU_TABLE), (la.ACT_Q8_1, la.GELU_TANH)])
+@pytest.mark.parametrize("T,chunks", [(2047, 1), (2048, 1), (2049, 2), (2300, 2), (4100, 3)])
+def test_prefill_longest_chunks(gpu, oracle, T, chunks, act_mode, gelu_mode):
+    """Around and past 16384 routed pairs (top-8: 2048 tokens): one full chunk,
+    two and three chunks of equal 64-token multiples with a short last one
+    (1088 + 961, 1152 + 1148, 1408 + 1408 + 1284).  The bias puts every token
+    on two experts (2048 pairs each: tens of groups) and leaves the rest
+    uneven.  Ids and weights against the oracle's router, outputs against its
+    experts, the routing counters against the ids.
+
+    A flipped q8 value moves by amax / 127 of its block, amax up to about 5
+    times the values' root mean square: 5 / (127 sqrt(N)) of a token that sums
+    N values of one weight.  Here the eight weights count for six (1 / sum of
+    their squares), three in the most uneven token: 1.4e-3 and 2.0e-3 at n_ff
+    128, within the bars' 3e-3.  (Two experts with all the weight and n_ff
+    64 would make it 3.5e-3.)"""
+    torch = torch_mod()
+    spec = la.LayerSpec(d_model=256, n_ff=128, n_expert=24, top_k=8)
+    say(f"prefill longest chunks T={T} act={act_mode}")
+    bias = np.linspace(0, 1, spec.n_expert).astype(np.float32)
+    bias[[2, 21]] = 2.0
+    lay = layer(spec, 620, [2, 5, 9, 20, 23], scales=True, router_bias=bias)
+    dl = la.DeviceLayer(lay, gpu, act_mode, gelu_mode)
+    dl.route_counts = torch.zeros(spec.n_expert, dtype=torch.int32, device=gpu)
+    dl.route_hits = torch.zeros(2, dtype=torch.int32, device=gpu)
+    x = tokens(621 + T, T, spec.d_model)
+    (out, ids, w), n = _chunks(dl, torch.from_numpy(x).to(gpu))
+    assert n == chunks
+    ids_g, w_g, out_g = ids.cpu().numpy(), w.cpu().numpy(), out.cpu().numpy()
+    ids_o, w_o, _ = oracle.router(x, lay.router_w, lay.router_b, spec.top_k)
+    assert np.array_equal(ids_g, ids_o)
+    assert np.allclose(w_g, w_o, rtol=1e-5, atol=1e-7)
+    counts = np.bincount(ids_g.ravel(), minlength=spec.n_expert)
+    assert counts.max() == T
+    hot = sum(int(c) for e, c in enumerate(counts) if lay.residency.is_hot(e))
+    assert np.array_equal(dl.route_counts.cpu().numpy(), counts)
+    assert dl.route_hits.tolist() == [hot, T * spec.top_k - hot]
+    want, _ = oracle.moe_experts(lay, x, ids_g, w_g, oracle_mode(act_mode, T), gelu_mode)
+    if act_mode == la.ACT_CPU:
+        check_flip_tolerant(out_g, want)
+    else:
+        check_layer_bars(out_g, want, say, 0.02)
 
 
 @pytest.mark.parametrize("n_ff", [32, 64, 96, 224, 320])

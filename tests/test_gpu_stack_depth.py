@@ -1,8 +1,8 @@
 """Config 5 at full depth: the 30-layer stack, h += moe(rms_norm(h)) per
 layer, in both activation modes -- decode (16 sequences of 1 token and 4 of
 4 tokens, one llapis call per sequence and layer) and a 530-token prefill (two
-chunks of at most 4096 routed pairs) -- against the oracle's own 30-layer
-chain.
+chunks of at most 4096 routed pairs, in a workspace sized for 512 tokens) --
+against the oracle's own 30-layer chain.
 
 Every layer has its own router (seeded per layer), its own Zipf(1.1) hot set
 of K = 57 experts with a router bias that puts ~85 % of the picks on it, and
@@ -54,7 +54,7 @@ import numpy as np
 import pytest
 
 import llapis_amd as la
-from helpers import FULL, full_layer, oracle_mode, per_token_rel_l2, rel_l2, tokens
+from helpers import FULL, full_layer, in_workspace_for, oracle_mode, per_token_rel_l2, rel_l2, tokens
 
 pytestmark = pytest.mark.gpu
 
@@ -154,9 +154,10 @@ def _flips(ids_a, ids_b):
     return np.array(out), gone
 
 
-def _run(gpu, oracle, calls, act_mode, gelu_mode, check_every, subset):
+def _run(gpu, oracle, calls, act_mode, gelu_mode, check_every, subset, ws_tokens=None):
     """calls: (first token, token count) of each llapis call per layer over
-    the input rows; subset: the rows the chains are compared on."""
+    the input rows; subset: the rows the chains are compared on; ws_tokens:
+    the tokens the calls' workspace is sized for (None: the call's own)."""
     import torch
     layers = _stack()
     n_rows = sum(c for _, c in calls)
@@ -167,6 +168,8 @@ def _run(gpu, oracle, calls, act_mode, gelu_mode, check_every, subset):
     for il, lay in enumerate(layers):
         xl = torch.nn.functional.rms_norm(h, (FULL.d_model,), eps=1e-6).contiguous()
         dl = la.DeviceLayer(lay, gpu, act_mode, gelu_mode)
+        if ws_tokens is not None:
+            in_workspace_for(dl, ws_tokens)
         outs, idss, ws = [], [], []
         for b, c in calls:
             o, i, w = dl.forward(xl[b:b + c])
@@ -251,8 +254,9 @@ def test_stack_full_depth_decode(gpu, oracle, act_mode, gelu_mode):
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("act_mode,gelu_mode", MODES)
 def test_stack_full_depth_prefill_two_chunks(gpu, oracle, act_mode, gelu_mode):
-    """One 530-token call per layer (4240 routed pairs: two chunks); the
-    chains compared on 64 rows spread over both chunks."""
+    """One 530-token call per layer (4240 routed pairs) in a workspace sized
+    for 512 tokens: chunks of 512 and 18.  The chains compared on 64 rows
+    spread over both chunks."""
     say(f"workload stack 30 layers prefill T=530 act={act_mode}")
     subset = np.unique(np.linspace(0, 529, 64).astype(int))
-    _run(gpu, oracle, [(0, 530)], act_mode, gelu_mode, 5, subset)
+    _run(gpu, oracle, [(0, 530)], act_mode, gelu_mode, 5, subset, ws_tokens=512)

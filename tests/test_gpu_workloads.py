@@ -25,8 +25,8 @@ import numpy as np
 import pytest
 
 import llapis_amd as la
-from helpers import (FULL, check_layer_bars, dual_k57, full_layer, oracle_mode, per_token_rel_l2, rel_l2, tokens,
-                     with_hot_set)
+from helpers import (FULL, check_layer_bars, dual_k57, full_layer, in_workspace_for, oracle_mode, per_token_rel_l2,
+                     rel_l2, tokens, with_hot_set)
 
 pytestmark = pytest.mark.gpu
 
@@ -92,8 +92,8 @@ def test_decode_dual_k57_four_tokens_per_token(gpu, oracle, act_mode, gelu_mode)
 @pytest.mark.parametrize("act_mode,gelu_mode", MODES)
 def test_prefill_dual_k57_512_tokens(gpu, oracle, act_mode, gelu_mode):
     """Config 4: a 512-token prefill chunk of the dual layer (4096 routed
-    pairs: the largest chunk the prefill path takes at top-8), bucketed by
-    expert into uneven groups."""
+    pairs: the shortest that a longer call is cut into), bucketed by expert
+    into uneven groups."""
     say(f"workload prefill dual K=57 T=512 act={act_mode}")
     lay = dual_k57(full_layer(SEED), 7)
     x = tokens(990, 512, FULL.d_model)
@@ -117,7 +117,8 @@ def _rms_norm_np(h, eps=1e-6):
 @pytest.mark.parametrize("act_mode,gelu_mode", MODES)
 @pytest.mark.parametrize("T", [1, 530])
 def test_stack_slice_three_layers(gpu, oracle, T, act_mode, gelu_mode):
-    """Config 5, three layers of the stack: h += moe(rms_norm(h)).  Each
+    """Config 5, three layers of the stack: h += moe(rms_norm(h)); 530 tokens
+    in a workspace sized for 512 (chunks of 512 and 18).  Each
     layer against the oracle on the GPU's own input to it (ids identical,
     within the layer bars), then the oracle's own chain (numpy RMSNorm and
     add) against the GPU's final residual stream: tokens routed alike in every
@@ -137,7 +138,7 @@ def test_stack_slice_three_layers(gpu, oracle, T, act_mode, gelu_mode):
     for il, lay in enumerate(layers):
         xl = torch.nn.functional.rms_norm(h, (FULL.d_model,), eps=1e-6)
         x = xl.cpu().numpy()
-        dl = la.DeviceLayer(lay, gpu, act_mode, gelu_mode)
+        dl = in_workspace_for(la.DeviceLayer(lay, gpu, act_mode, gelu_mode), min(T, 512))
         out, ids, w = dl.forward(xl.contiguous())
         torch.cuda.synchronize()
         ids_g, w_g, out_g = ids.cpu().numpy(), w.cpu().numpy(), out.cpu().numpy()
