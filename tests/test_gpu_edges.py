@@ -6,6 +6,7 @@ READY slot whose slot_exp points back at the expert is hot).  Each case runs
 the decode path (1 and 3 tokens) and the prefill path (40 tokens), in the
 CPU-parity activation mode and in the q8_1 mode."""
 import copy
+import dataclasses
 
 import numpy as np
 import pytest
@@ -97,6 +98,48 @@ def test_prefill_wide_model(gpu, oracle, act_mode, gelu_mode):
         check_flip_tolerant(out.cpu().numpy(), out_o)
     else:
         check_layer_bars(out.cpu().numpy(), out_o, say, 0.02)
+
+
+def _formats_layer(spec, hot, tiers):
+    """A layer whose hot / cold pools hold the formats `tiers` names: 0 is
+    Q4_K and Q5_0, 1 is IQ2_S and IQ4_NL."""
+    base = layer(spec, 740, list(range(spec.n_expert)), scales=True)
+    pools = [(la.Q4_K, la.Q5_0, base.hot_gu, base.hot_dn), (la.IQ2_S, la.IQ4_NL, base.cold_gu, base.cold_dn)]
+    lay = copy.copy(base)
+    (hg, hd, hot_gu, hot_dn), (cg, cd, lay.cold_gu, lay.cold_dn) = pools[tiers[0]], pools[tiers[1]]
+    lay.spec = dataclasses.replace(spec, hot_gu_type=hg, hot_dn_type=hd, cold_gu_type=cg, cold_dn_type=cd)
+    gb, db = spec.gu_bytes(hg), spec.dn_bytes(hd)
+    lay.hot_gu = np.concatenate([hot_gu[e * gb:(e + 1) * gb] for e in hot])
+    lay.hot_dn = np.concatenate([hot_dn[e * db:(e + 1) * db] for e in hot])
+    lay.s_hot = base.s_hot[hot].copy()
+    lay.residency = la.Residency.from_hot(spec.n_expert, hot)
+    return lay
+
+
+@pytest.mark.parametrize("act_mode,gelu_mode", [(la.ACT_CPU, la.GELU_TABLE), (la.ACT_Q8_1, la.GELU_TANH)])
+@pytest.mark.parametrize("T", [1, 3, 40, 150])
+@pytest.mark.parametrize("tiers", [(1, 0), (0, 0), (1, 1)])
+def test_formats_in_either_tier(gpu, oracle, tiers, T, act_mode, gelu_mode):
+    """The formats swapped between the tiers, and one pair of formats in both:
+    kernels of their own in the decode and prefill paths.  n_ff 192 (down rows
+    of three block pairs), d_model 768 (three super-blocks), groups of one to
+    several tiles."""
+    torch = torch_mod()
+    spec = LayerSpec(d_model=768, n_ff=192, n_expert=12, top_k=4)
+    say(f"formats tiers={tiers} T={T} act={act_mode}")
+    lay = _formats_layer(spec, [1, 4, 6, 9, 11], tiers)
+    dl = la.DeviceLayer(lay, gpu, act_mode, gelu_mode)
+    x = tokens(741 + T, T, spec.d_model)
+    out, ids, w = dl.forward(torch.from_numpy(x).to(gpu))
+    ids_g, w_g, out_g = ids.cpu().numpy(), w.cpu().numpy(), out.cpu().numpy()
+    ids_o, w_o, _ = oracle.router(x, lay.router_w, lay.router_b, spec.top_k)
+    assert np.array_equal(ids_g, ids_o)
+    assert np.allclose(w_g, w_o, rtol=1e-5, atol=1e-7)
+    want, _ = oracle.moe_experts(lay, x, ids_g, w_g, oracle_mode(act_mode, T), gelu_mode)
+    if T > 4 and act_mode == la.ACT_Q8_1:
+        check_layer_bars(out_g, want, say, 0.02)
+    else:
+        check_flip_tolerant(out_g, want)
 
 
 def test_zero_tokens_is_a_no_op(gpu):
