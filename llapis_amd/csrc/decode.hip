@@ -632,8 +632,10 @@ void k_dec_gate_up(const DecParams p) {
     constexpr bool IQ2 = HT == T_IQ2_S || CT == T_IQ2_S;
     constexpr int COLL = MT == 1 ? 1 : 2;                 // quantised column chunks per thread issued at once
     constexpr int TABL = (TAB_CHUNKS + GU_NT - 1) / GU_NT;   // codebook chunks per thread
-    // the routing's scratch lives where the weights are staged later (the
-    // first item starts with a barrier, after every read of it)
+    // the routing's scratch lives where the weights are staged later: the
+    // barrier after build_groups is what ends it (the first item's copies start
+    // right after that barrier, with no other between), and it publishes the
+    // columns and the codebook too.  Nothing may read the scratch past it.
     GuScratch & sr = *reinterpret_cast<GuScratch *>(smem);
     __shared__ int s_ids[DEC_PMAX];           // the routing, kept past the scratch's reuse
     __shared__ float s_w[DEC_PMAX];
@@ -678,7 +680,7 @@ void k_dec_gate_up(const DecParams p) {
     // every token's quantised column (contiguous: xq_stride == their size) and
     // the IQ2_S codebook: they do not depend on the routing, so they are in LDS
     // (after the two halves: at a0) before the first weights are asked for, and
-    // the routing's last barrier publishes them (read after the routing, before
+    // the routing's barriers publish them (read after the routing, before
     // the weights, they cost a one-token layer 1.0 of 24.5 us, a four-token one
     // 1.7 of 39.9)
     ActView tmp;
@@ -750,7 +752,7 @@ void k_dec_gate_up(const DecParams p) {
         return validate_group(p, gi, ng, g);
     };
 
-    // 3. the first item's weights (the routing's scratch is dead: the barrier above)
+    // 3. the first item's weights, into the scratch's room (dead since the barrier above)
     int it = blockIdx.x, j, h = 0;
     GroupInfo gi = item(it, &j);
     gu_wave_load<HT, CT, MT>(p, gi, j, 0, smem);
@@ -1021,17 +1023,22 @@ __device__ __forceinline__ void q8_quad(uint8_t * col, const ActView & L, const 
 }
 
 // C: output rows [r0, r0 + R) of every token, r0 = blockIdx.x R, R =
-// 2^dn_rows_log2.  First, with no dependence on anything, the loads of the
-// pairs' quantised down columns (written by B; the pairs are 0 .. T top_k - 1
-// whatever the grouping) and of the groups' records and routing weights
-// (from B's first workgroup); then a table of the groups (tier, members,
-// .scale, where this block's rows start in the pool).  The weights never
-// pass through LDS: each row's lanes load its block pairs straight into
-// registers (lane l: blocks 2 l, 2 l + 1, dword-aligned), the next pass's
-// rows in flight while the current ones are dotted against the members'
-// columns in LDS.  Each row is scaled by the expert's .scale into
-// s_y[pair][row]; then each (token, row) output is the sum of w_k y_k in k
-// order.  Invalid groups leave their pairs at zero.
+// 2^dn_rows_log2.  Inputs: the pairs' quantised down columns (written by B;
+// the pairs are 0 .. T top_k - 1 whatever the grouping) and the groups'
+// records and routing weights (from B's first workgroup).  A table of the
+// groups in LDS holds tier, members, .scale and where this block's rows start
+// in the pool.  The weights never pass through LDS: each row's lanes load its
+// block pairs straight into registers (lane l: blocks 2 l, 2 l + 1,
+// dword-aligned), several passes in flight (DA), and dot them against the
+// members' columns in LDS.
+//   One token (MT == 1): every lane reads its own passes' records and starts
+//   its rows from them, before any barrier; the table and the columns go to
+//   LDS meanwhile, one barrier publishes both.
+//   2-4 tokens: the columns' loads, then the table (a barrier each side),
+//   then the rows from the table, the columns into LDS, a barrier.
+// Each row is scaled by the expert's .scale into s_y[pair][row]; then each
+// (token, row) output is the sum of w_k y_k in k order.  Invalid groups leave
+// their pairs at zero.
 template <int HD, int CD, int AM, int MT>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(1, 4))) void k_dec_down(const DecParams p) {
     extern __shared__ __align__(16) uint8_t smem[];
