@@ -128,10 +128,10 @@ hipError_t launch_fire(const FireParams & f, int ht, int ct, int act_mode, hipSt
 
 constexpr int PF_ROWS = 128;          // weight rows per workgroup (4 waves x 32)
 constexpr int PF_TOK = 64;            // routed pairs per down group (four 16-token MFMA tiles)
-constexpr int PF_GTOK = 128;          // routed pairs per gate_up group, at most
+constexpr int PF_GTOK = 48;           // routed pairs per gate_up group, at most (three 16-token MFMA tiles)
 constexpr int PF_MAX_PAIRS = 16384;   // routed pairs per prefill launch (T * top_k), at most
 constexpr int PF_MIN_PAIRS = 4096;    // ... that a workspace of any accepted size holds
-constexpr int PF_MAX_FF = 4096;       // longest n_ff the down activation kernel stages
+constexpr int PF_MAX_FF = 4096;       // longest n_ff of the prefill path
 
 // a group: a run of up to PF_TOK pairs routed to one expert
 struct PfTile {
@@ -152,7 +152,7 @@ struct PfParams {
     const uint8_t * cold_dn; uint64_t cold_dn_stride;
     const float * s_hot; const float * s_cold;
     int * n_tiles;                       // [1]
-    int32_t * sorted;                    // [P] pair indices grouped by expert, ascending within
+    int32_t * sorted;                    // [P] pair indices grouped by expert, in any order within
     PfTile * tiles;                      // [max_tiles]
     int max_tiles;
     // the gate_up kernel's groups: runs of up to gcap[tier] pairs of one
@@ -160,7 +160,7 @@ struct PfParams {
     PfTile * gtiles;                     // [max_gtiles]
     int * n_gtiles;                      // [1]
     int max_gtiles;
-    int gcap[2];                         // hot, cold (a multiple of 16 in [16, PF_GTOK])
+    int gcap[2];                         // hot, cold (16, 32 or 48)
     int8_t * xq;                         // [T][d_model] q8_K values
     float * xd;                          // [T][d_model / 256] q8_K scales
     _Float16 * xm;                       // [T][d_model / 256][16] q8_K: per-32 sums as 32 hi + lo;
@@ -175,6 +175,7 @@ struct PfParams {
 };
 
 int pf_max_tiles(int P, int n_expert);
+// room for groups of 16 pairs, the shortest the bucketing makes full groups of
 int pf_max_gtiles(int P, int n_expert);
 // ev (optional, profiling): begin/end timestamps of the gate_up and down GEMMs
 hipError_t launch_prefill(const PfParams & p, int hgu, int cgu, int hdn, int cdn, int gelu_src, hipStream_t s,

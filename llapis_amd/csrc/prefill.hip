@@ -445,7 +445,7 @@ __device__ __forceinline__ void q8_store32(float v, _Float16 * hi, _Float16 * lo
 // meet no bank conflict.
 
 constexpr int G2_TOK = 48;              // pairs per group (three 16-token MFMA tiles)
-static_assert(G2_TOK <= PF_GTOK, "group cap");
+static_assert(G2_TOK == PF_GTOK, "group cap");
 constexpr int G2_MBT = (G2_TOK + 31) / 32 * 32;       // tokens of a mins buffer: 32 per moving wave
 
 // LDS of one workgroup.  Each of the two buffers of a kind is a separate
@@ -967,6 +967,7 @@ __constant__ Iq2sHalf c_iq2s_half = make_iq2s_half();
 constexpr int PF_XH = 512 + 8;            // halfs per staged token row of one super-block: 256 hi, 256 lo, pad
 constexpr int PF_TOK1Q4 = 48;             // pairs per gate_up group in the q8_1 mode, Q4_K expert
 constexpr int PF_TOK1IQ2 = 32;            // IQ2_S expert (its tables take the room of 16 tokens)
+static_assert(PF_TOK1Q4 <= PF_GTOK && PF_TOK1IQ2 <= PF_GTOK, "group caps");
 constexpr int GU1_XREG = 4;               // activation chunks per thread per super-block and 16-token tile (16 x 64)
 
 // The LDS of one workgroup.  An IQ2_S group (its rows go straight to
