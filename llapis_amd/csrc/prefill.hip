@@ -436,7 +436,7 @@ __device__ __forceinline__ void q8_store32(float v, _Float16 * hi, _Float16 * lo
 // into the same room, so one buffer is enough and three workgroups share a CU
 // instead of two (the kernel is bound by VALU issue and, between a
 // workgroup's steps, by waits that other workgroups fill: fastest traced
-// dispatches 126 -> 110 us at 512 tokens, dual K = 57, 283 -> 236 us at 1900
+// dispatches 126 -> 110 us at 512 tokens, dual K = 57, 283 -> 242 us at 1900
 // tokens, all hot, 40 -> 36 us at 12 tokens).  IQ2_S rows, read straight into
 // registers before, came in 64 accesses of the L1 a 12-byte load: through the
 // windows 110 -> 105 us at 512 tokens, 36 -> 32 us at 12.  A token's 16-byte chunk c of a
@@ -1339,9 +1339,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // 512-token chunk (dual, K = 57), 240 thousand of a CU's 290 thousand cycles.
 // With the windows in LDS 16 million, and with the fragment order of dn_pos
 // and dn_frag's fewer VALU instructions (27 against 35 million) the kernel
-// takes 92 against 122 us there (fastest dispatches, traced), 211 against 254
-// us at 1900 tokens, 26 against 34 us at 12.  It is bound by VALU issue (57 %
-// of its cycles) and the matrix cores (21 %).  Groups of 64 pairs: at 96 the
+// takes 90 against 122 us there (fastest dispatches, traced), 214 against 254
+// us at 1900 tokens, 27 against 34 us at 12.  It is bound by VALU issue (58 %
+// of its cycles there) and the matrix cores (21 %).  Groups of 64 pairs: at 96 the
 // activation buffers leave room for two workgroups a CU instead of three.
 constexpr int D2_XB = PF_TOK * 256;                // activations of one step: [chunk][pair slot][16][16 bytes]
 constexpr int D2_WB = 4 * 1024;                    // one wave's weight windows of a step, at most (whole copies)
