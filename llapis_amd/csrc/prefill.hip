@@ -444,7 +444,12 @@ __device__ __forceinline__ void q8_store32(float v, _Float16 * hi, _Float16 * lo
 // tokens of an MFMA fragment read 16 distinct slots, so the fragment loads
 // meet no bank conflict.
 
-constexpr int G2_TOK = 48;              // pairs per group (three 16-token MFMA tiles)
+// Pairs per group (three 16-token MFMA tiles), of either format.  IQ2_S groups
+// of 64, which leave two workgroups a CU, are behind where every expert is
+// cold too, though a full group's rows are then expanded less often (d_model
+// 2816, n_ff 704, top-8 of 128, the windows below included, medians: 64 tokens
+// 74 against 60 us, 173 tokens 91 / 71, 512 tokens 126 / 110).
+constexpr int G2_TOK = 48;
 static_assert(G2_TOK == PF_GTOK, "group cap");
 constexpr int G2_MBT = (G2_TOK + 31) / 32 * 32;       // tokens of a mins buffer: 32 per moving wave
 
