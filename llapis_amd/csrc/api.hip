@@ -672,8 +672,8 @@ bool decode_eligible(const llapis_moe_layer * L, int32_t T) {
 // chunks of Tc tokens; one chunk's scratch.  A chunk reads every routed
 // expert's weights, so a call is cut into as few chunks as PF_MAX_PAIRS and
 // the workspace allow, of equal size (whole 64-token router tiles): 1900
-// tokens at top-8, d_model 2816, every expert hot, take 1036 us as four
-// 512-token chunks and 566 us in one.  Chunks of PF_MIN_PAIRS / top_k tokens
+// tokens at top-8, d_model 2816, every expert hot, take 513 us in one chunk,
+// 614 in two, 754 in three and 888 in four.  Chunks of PF_MIN_PAIRS / top_k tokens
 // (the whole call, if it is shorter) are the shortest.
 struct PfWs {
     uint64_t probs, ids, w, ntiles, sorted, tiles, gtiles, xq, xd, xm, xh, ah, al, ydn, parts, total;
